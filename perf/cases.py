@@ -75,7 +75,7 @@ def draw(rng):
     batch = min(int(math.exp(rng.uniform(0.0, math.log(room + 0.99)))), 11) if order < top else rng.randint(1, 2)
     j = rng.randint(max(2, order - 3), order - 1)
     if kind == "eval" and order == top:
-        batch, j = 1, min(j, order - 2)  # with every scale it is a listed case
+        batch, j = 1, rng.randint(3, order - 2)  # with every scale it is a listed case
     case = {"kind": kind, "precision": precision, "nside": 1 << order, "j": j, "batch": batch}
     if kind == "masks":
         case["masks"] = rng.randint(1, 7)
