@@ -1402,7 +1402,7 @@ class EngineT final : public Engine {
       for (int n = qc_; n < levels_; ++n) {
         const int64_t N = N_[n];
         const ConvOp<T> conv = conv_[n]->store.view();
-        LevelTask<T> z = base(kQConvFwd1, n, B_, blocks(N * 8, 256));
+        LevelTask<T> z = base(kQConvFwd1, n, B_, split_blocks(N));
         z.conv = conv;
         z.in0 = f_->maps[n].data();
         z.out0 = f_->z[n].data();
@@ -1415,7 +1415,7 @@ class EngineT final : public Engine {
         d.in0 = f_->M[n - 1].data();
         d.out0 = f_->M[n].data();
         decs.push_back(Step{{d}, dec_bytes(n - 1, kL, n * B_), tag("batch_dec_fwd", n)});
-        LevelTask<T> b = base(kQConvFwd4, n, (n + 1) * B_, blocks(N * 8, 256));
+        LevelTask<T> b = base(kQConvFwd4, n, (n + 1) * B_, split_blocks(N));
         b.conv = conv;
         b.in0 = f_->M[n].data();
         b.out0 = f_->br[n].data();
@@ -1468,7 +1468,7 @@ class EngineT final : public Engine {
       v.out1 = f_->qgzp[n].data();
       vs.tasks.push_back(v);
       vs.bytes += double(B_) * N * ((n + 1) * kL * kL + kL) * 2 * sizeof(T) * 2;
-      LevelTask<T> a = base(kQConvAdj4, n, (n + 1) * B_, blocks(N * 8, 256));
+      LevelTask<T> a = base(kQConvAdj4, n, (n + 1) * B_, split_blocks(N));
       a.conv = conv;
       a.in0 = f_->qgbr[n].data();
       a.out0 = f_->qchain[n].data();
@@ -1499,7 +1499,7 @@ class EngineT final : public Engine {
       z.out0 = f_->qgz[n].data();
       zs.tasks.push_back(z);
       zs.bytes += double(B_) * kL * N * (7 * sizeof(T));
-      LevelTask<T> za1 = base(kQConvAdj1, n, B_, blocks(N * 8, 256));
+      LevelTask<T> za1 = base(kQConvAdj1, n, B_, split_blocks(N));
       za1.conv = conv;
       za1.in0 = f_->qgz[n].data();
       za1.out0 = f_->qmg[n].data();

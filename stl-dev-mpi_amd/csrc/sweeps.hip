@@ -187,10 +187,20 @@ __global__ __launch_bounds__(256) void k_conv_adj(ConvOp<T> op, const cplx_t<T>*
 // The same gathers with the slots of one output spread over LP consecutive
 // lanes, for levels too small to fill the GPU: each thread's chain of
 // dependent loads is LP times shorter.  The LP partial sums are added by a
-// fixed butterfly (deterministic).
+// fixed butterfly (deterministic).  What bounds them is that chain, about 1 us
+// a memory latency: with NI = 1 a lane loads the ids of 4 slots together with
+// the row's count, then their coefficients and inputs together (NI = kL holds
+// too many values for that; its loop takes a slot at a time).
 // Bodies of the 256-thread kernels take their block (bx, row) as arguments, so
-// that the work-queue kernel of the coarse levels can run them as items.
-template <typename T, int NI, int LP>
+// that the batched launches of the coarse levels can run them as items.
+constexpr int kSplitLanes = 8, kSplitChunk = 4;
+// The per-level kernels' slots go in chunks in FP64 only: they are candidates
+// of the variant timing, and in FP32 a split level's sums round in another
+// order than the tiled variants', so the engines keep the choices they had.
+template <typename T>
+constexpr bool kSplitChunked = sizeof(T) == 8;
+
+template <typename T, int NI, int LP, bool CHUNKED>
 __device__ __forceinline__ void conv_fwd_split_body(const ConvOp<T>& op, const T* __restrict__ x,
                                                     cplx_t<T>* __restrict__ y, T* __restrict__ mod, int64_t bx,
                                                     int row) {
@@ -208,22 +218,60 @@ __device__ __forceinline__ void conv_fwd_split_body(const ConvOp<T>& op, const T
 #pragma unroll
     for (int g = 0; g < kL; ++g) acc[j][g][0] = acc[j][g][1] = T(0);
   const int cnt = active ? op.cnt[r] : 0;
-  for (int s = lane; s < cnt; s += LP) {
-    size_t at = size_t(s) * op.R + r;
-    int64_t ck = rot_pix(op.cell[at], k, op.order);
-    if (mir) ck = mirror_pix(ck, op.order);
-    T c[8], a[8];
-    Load<T>::coef8(op.coef + at * 8, c);
-    permute<T>(k, c, a);
-    T xv[NI];
-    Load<T>::template vec<NI>(xr + size_t(ck) * NI, xv);
+  if constexpr (NI == 1 && CHUNKED) {
+    for (int c0 = lane; c0 < op.S; c0 += kSplitChunk * LP) {
+      int32_t ck[kSplitChunk];
+      T c[kSplitChunk][8], xv[kSplitChunk];
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int g = 0; g < kL; ++g) {
-        acc[j][g][0] += a[g * 2] * xv[j];
-        acc[j][g][1] += a[g * 2 + 1] * xv[j];
+      for (int u = 0; u < kSplitChunk; ++u) {
+        const size_t at = size_t(min(c0 + u * LP, op.S - 1)) * op.R + r;
+        ck[u] = op.cell[at];
+        Load<T>::coef8(op.coef + at * 8, c[u]);
       }
+      // Past the count a slot reads cell 0 and adds 0 * 0 (by selection: a
+      // branch would draw the loads into it).
+#pragma unroll
+      for (int u = 0; u < kSplitChunk; ++u) {
+        int64_t cell = rot_pix(c0 + u * LP < cnt ? ck[u] : 0, k, op.order);
+        if (mir) cell = mirror_pix(cell, op.order);
+        xv[u] = xr[cell];
+      }
+#pragma unroll
+      for (int u = 0; u < kSplitChunk; ++u) {
+        const bool in = c0 + u * LP < cnt;
+        T a[8];
+#pragma unroll
+        for (int g = 0; g < kL; ++g) {
+          const T re = k & 1 ? c[u][(g ^ 2) * 2] : c[u][g * 2], im = k & 1 ? c[u][(g ^ 2) * 2 + 1] : c[u][g * 2 + 1];
+          a[g * 2] = in ? re : T(0);
+          a[g * 2 + 1] = in ? (gauge_conj(k, g) ? -im : im) : T(0);
+        }
+        const T xu = in ? xv[u] : T(0);
+#pragma unroll
+        for (int g = 0; g < kL; ++g) {
+          acc[0][g][0] = fma(a[g * 2], xu, acc[0][g][0]);
+          acc[0][g][1] = fma(a[g * 2 + 1], xu, acc[0][g][1]);
+        }
+      }
+    }
+  } else {
+    for (int s = lane; s < cnt; s += LP) {
+      size_t at = size_t(s) * op.R + r;
+      int64_t ck = rot_pix(op.cell[at], k, op.order);
+      if (mir) ck = mirror_pix(ck, op.order);
+      T c[8], a[8];
+      Load<T>::coef8(op.coef + at * 8, c);
+      permute<T>(k, c, a);
+      T xv[NI];
+      Load<T>::template vec<NI>(xr + size_t(ck) * NI, xv);
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int g = 0; g < kL; ++g) {
+          acc[j][g][0] += a[g * 2] * xv[j];
+          acc[j][g][1] += a[g * 2 + 1] * xv[j];
+        }
+    }
   }
 #pragma unroll
   for (int m = LP / 2; m >= 1; m >>= 1)
@@ -251,10 +299,10 @@ __device__ __forceinline__ void conv_fwd_split_body(const ConvOp<T>& op, const T
 template <typename T, int NI, int LP>
 __global__ __launch_bounds__(256) void k_conv_fwd_split(ConvOp<T> op, const T* __restrict__ x,
                                                         cplx_t<T>* __restrict__ y, T* __restrict__ mod) {
-  conv_fwd_split_body<T, NI, LP>(op, x, y, mod, blockIdx.x, blockIdx.y);
+  conv_fwd_split_body<T, NI, LP, kSplitChunked<T>>(op, x, y, mod, blockIdx.x, blockIdx.y);
 }
 
-template <typename T, int NI, int LP>
+template <typename T, int NI, int LP, bool CHUNKED>
 __device__ __forceinline__ void conv_adj_split_body(const ConvOp<T>& op, const cplx_t<T>* __restrict__ gy,
                                                     T* __restrict__ gx, int64_t bx, int row) {
   const int64_t o = (bx * 256 + threadIdx.x) / LP;
@@ -269,25 +317,58 @@ __device__ __forceinline__ void conv_adj_split_body(const ConvOp<T>& op, const c
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
   const int cnt = active ? op.tcnt[q] : 0;
-  for (int s = lane; s < cnt; s += LP) {
-    size_t at = size_t(s) * op.R + q;
-    int64_t pk = rot_pix(op.trow[at], k, op.order);
-    if (mir) pk = mirror_pix(pk, op.order);
-    T c[8], a[8];
+  if constexpr (NI == 1 && CHUNKED) {
+    const cplx_t<T>* tc = reinterpret_cast<const cplx_t<T>*>(op.tcoef) + q;
+    for (int c0 = lane; c0 < op.Tn; c0 += kSplitChunk * LP) {
+      int32_t pk[kSplitChunk];
+      cplx_t<T> c[kSplitChunk][kL], v[kSplitChunk][kL];
 #pragma unroll
-    for (int g = 0; g < kL; ++g) {
-      cplx_t<T> v = reinterpret_cast<const cplx_t<T>*>(op.tcoef)[(size_t(g) * op.Tn + s) * op.R + q];
-      c[2 * g] = v.x;
-      c[2 * g + 1] = mir ? -v.y : v.y;
+      for (int u = 0; u < kSplitChunk; ++u) {
+        const int s = min(c0 + u * LP, op.Tn - 1);
+        pk[u] = op.trow[size_t(s) * op.R + q];
+        // Gauge g of face shift k reads the coefficient plane gauge_src(k, g).
+#pragma unroll
+        for (int g = 0; g < kL; ++g) c[u][g] = tc[(size_t(gauge_src(k, g)) * op.Tn + s) * op.R];
+      }
+#pragma unroll
+      for (int u = 0; u < kSplitChunk; ++u) {
+        int64_t row_pix = rot_pix(c0 + u * LP < cnt ? pk[u] : 0, k, op.order);
+        if (mir) row_pix = mirror_pix(row_pix, op.order);
+#pragma unroll
+        for (int g = 0; g < kL; ++g) v[u][g] = gr[size_t(g) * N + row_pix];
+      }
+#pragma unroll
+      for (int u = 0; u < kSplitChunk; ++u) {
+        const bool in = c0 + u * LP < cnt;
+#pragma unroll
+        for (int g = 0; g < kL; ++g) {
+          const T cx = in ? c[u][g].x : T(0);
+          const T cy = in ? (gauge_conj(k, g) != mir ? -c[u][g].y : c[u][g].y) : T(0);
+          acc[0] = fma(cy, in ? v[u][g].y : T(0), fma(cx, in ? v[u][g].x : T(0), acc[0]));
+        }
+      }
     }
-    permute<T>(k, c, a);
+  } else {
+    for (int s = lane; s < cnt; s += LP) {
+      size_t at = size_t(s) * op.R + q;
+      int64_t pk = rot_pix(op.trow[at], k, op.order);
+      if (mir) pk = mirror_pix(pk, op.order);
+      T c[8], a[8];
 #pragma unroll
-    for (int g = 0; g < kL; ++g) {
-      const cplx_t<T>* src = gr + (size_t(g) * N + pk) * NI;
+      for (int g = 0; g < kL; ++g) {
+        cplx_t<T> v = reinterpret_cast<const cplx_t<T>*>(op.tcoef)[(size_t(g) * op.Tn + s) * op.R + q];
+        c[2 * g] = v.x;
+        c[2 * g + 1] = mir ? -v.y : v.y;
+      }
+      permute<T>(k, c, a);
 #pragma unroll
-      for (int j = 0; j < NI; ++j) {
-        cplx_t<T> v = src[j];
-        acc[j] = fma(a[g * 2 + 1], v.y, fma(a[g * 2], v.x, acc[j]));
+      for (int g = 0; g < kL; ++g) {
+        const cplx_t<T>* src = gr + (size_t(g) * N + pk) * NI;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          cplx_t<T> v = src[j];
+          acc[j] = fma(a[g * 2 + 1], v.y, fma(a[g * 2], v.x, acc[j]));
+        }
       }
     }
   }
@@ -305,7 +386,7 @@ __device__ __forceinline__ void conv_adj_split_body(const ConvOp<T>& op, const c
 template <typename T, int NI, int LP>
 __global__ __launch_bounds__(256) void k_conv_adj_split(ConvOp<T> op, const cplx_t<T>* __restrict__ gy,
                                                         T* __restrict__ gx) {
-  conv_adj_split_body<T, NI, LP>(op, gy, gx, blockIdx.x, blockIdx.y);
+  conv_adj_split_body<T, NI, LP, kSplitChunked<T>>(op, gy, gx, blockIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1182,12 +1263,40 @@ constexpr int kDecPre = 8;
 
 template <typename T>
 __device__ inline void dec_prefetch(const int16_t* __restrict__ off, const T* __restrict__ val, int64_t R, int cap,
-                                    int64_t r, int cnt, int16_t (&eo)[kDecPre], T (&ev)[kDecPre]) {
+                                    int64_t r, int cnt, int s0, int16_t (&eo)[kDecPre], T (&ev)[kDecPre]) {
 #pragma unroll
-  for (int s = 0; s < kDecPre; ++s) {
-    const size_t at = size_t(min(s, cap - 1)) * R + r;
-    eo[s] = off[at];
-    ev[s] = s < cnt ? val[at] : T(0);
+  for (int u = 0; u < kDecPre; ++u) {
+    const size_t at = size_t(min(s0 + u, cap - 1)) * R + r;
+    eo[u] = off[at];
+    ev[u] = s0 + u < cnt ? val[at] : T(0);
+  }
+}
+
+// Sum of a row's entries over its staged window (planes of PLANE elements,
+// rows of SW): the first kDecPre entries are in eo / ev; each further chunk
+// loads while the previous one's products run (an entry at a time, its load
+// was waited for before the next one's was issued).
+template <typename T, int NI, int SW, int PLANE>
+__device__ __forceinline__ void dec_gather(const int16_t* __restrict__ off, const T* __restrict__ val, int64_t R,
+                                           int cap, int64_t r, int cnt, int16_t (&eo)[kDecPre], T (&ev)[kDecPre],
+                                           const T* xs, int pos, T (&acc)[NI]) {
+  for (int s0 = 0;; s0 += kDecPre) {
+    int16_t no[kDecPre];
+    T nv[kDecPre];
+    // Unconditional (slots clamped to the capacity), as in pipelined_slots.
+    dec_prefetch<T>(off, val, R, cap, r, cnt, s0 + kDecPre, no, nv);
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) {
+      const int src = pos + off_dy(eo[u]) * SW + off_dx(eo[u]);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[j] = fma(ev[u], xs[j * PLANE + src], acc[j]);
+    }
+    if (s0 + kDecPre >= cnt) return;
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) {
+      eo[u] = no[u];
+      ev[u] = nv[u];
+    }
   }
 }
 
@@ -1229,7 +1338,7 @@ __global__ __launch_bounds__(TC * TC) void k_dec_fwd_tiled(DecOp<T> op, const T*
   const int cnt = op.cnt[r];
   int16_t eo[kDecPre];
   T ev[kDecPre];
-  dec_prefetch<T>(op.off, op.val, op.Rc, op.S, r, cnt, eo, ev);
+  dec_prefetch<T>(op.off, op.val, op.Rc, op.S, r, cnt, 0, eo, ev);
   const bool inside = span_inside(fx0, fy0, SW, op.order_f);
   stage_window<T, NI, SA, SA, TC * TC>(xr, xs, [&](int idx, int& lp) {
     int wx, wy;
@@ -1244,20 +1353,7 @@ __global__ __launch_bounds__(TC * TC) void k_dec_fwd_tiled(DecOp<T> op, const T*
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-#pragma unroll
-  for (int s = 0; s < kDecPre; ++s) {
-    const int src = pos + off_dy(eo[s]) * SW + off_dx(eo[s]);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += ev[s] * xs[j * SA + src];
-  }
-  for (int s = kDecPre; s < cnt; ++s) {
-    size_t at = size_t(s) * op.Rc + r;
-    int16_t o = op.off[at];
-    const T v = op.val[at];
-    const int src = pos + off_dy(o) * SW + off_dx(o);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += v * xs[j * SA + src];
-  }
+  dec_gather<T, NI, SW, SA>(op.off, op.val, op.Rc, op.S, r, cnt, eo, ev, xs, pos, acc);
   const int64_t p = int64_t(ti.face) * op.npf_c + ti.base + li;
 #pragma unroll
   for (int j = 0; j < NI; ++j) y[(size_t(row) * Nc + p) * NI + j] = acc[j];
@@ -1282,7 +1378,7 @@ __device__ __forceinline__ void dec_adj_tile(const DecOp<T>& op, const T* __rest
   const int cnt = op.tcnt[q];
   int16_t eo[kDecPre];
   T ev[kDecPre];
-  dec_prefetch<T>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, eo, ev);
+  dec_prefetch<T>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, 0, eo, ev);
   T base[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) base[j] = add ? add[o + j] : T(0);
@@ -1299,20 +1395,7 @@ __device__ __forceinline__ void dec_adj_tile(const DecOp<T>& op, const T* __rest
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-#pragma unroll
-  for (int s = 0; s < kDecPre; ++s) {
-    const int src = pos + off_dy(eo[s]) * SW + off_dx(eo[s]);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += ev[s] * gs[j * SA + src];
-  }
-  for (int s = kDecPre; s < cnt; ++s) {
-    size_t at = size_t(s) * op.Rf + q;
-    int16_t e = op.toff[at];
-    const T v = op.tval[at];
-    const int src = pos + off_dy(e) * SW + off_dx(e);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += v * gs[j * SA + src];
-  }
+  dec_gather<T, NI, SW, SA>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, eo, ev, gs, pos, acc);
 #pragma unroll
   for (int j = 0; j < NI; ++j) h[j] = add ? acc[j] + base[j] : acc[j];
 }
@@ -1331,6 +1414,33 @@ __global__ __launch_bounds__(TF * TF) void k_dec_adj_tiled(DecOp<T> op, const T*
   for (int j = 0; j < NI; ++j) gx[o + j] = h[j];
 }
 
+// Sum of a row's entries read through the caches, kDecPre at a time (ids and
+// weights together, then the inputs): two memory latencies per chunk.
+template <typename T, int NI>
+__device__ __forceinline__ void dec_gather_global(const int32_t* __restrict__ id, const T* __restrict__ val,
+                                                  int64_t R, int64_t r, int cnt, const T* __restrict__ xr, int k,
+                                                  int order, T (&acc)[NI]) {
+  for (int s0 = 0; s0 < cnt; s0 += kDecPre) {
+    int32_t ids[kDecPre];
+    T v[kDecPre], xv[kDecPre][NI];
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) {
+      const size_t at = size_t(min(s0 + u, cnt - 1)) * R + r;
+      ids[u] = id[at];
+      v[u] = val[at];
+    }
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) Load<T>::template vec<NI>(xr + size_t(rot_pix(ids[u], k, order)) * NI, xv[u]);
+    // Past the count 0 * 0: by selection, a branch would draw the loads into it.
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) {
+      const bool in = s0 + u < cnt;
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[j] = fma(in ? v[u] : T(0), in ? xv[u][j] : T(0), acc[j]);
+    }
+  }
+}
+
 template <typename T, int NI>
 __device__ __forceinline__ void dec_fwd_body(const DecOp<T>& op, const T* __restrict__ x, T* __restrict__ y,
                                              int64_t bx, int row) {
@@ -1344,16 +1454,7 @@ __device__ __forceinline__ void dec_fwd_body(const DecOp<T>& op, const T* __rest
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-  int cnt = op.cnt[r];
-  for (int s = 0; s < cnt; ++s) {
-    size_t at = size_t(s) * op.Rc + r;
-    int64_t fk = rot_pix(op.col[at], k, op.order_f);
-    T v = op.val[at];
-    T xv[NI];
-    Load<T>::template vec<NI>(xr + size_t(fk) * NI, xv);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += v * xv[j];
-  }
+  dec_gather_global<T, NI>(op.col, op.val, op.Rc, r, op.cnt[r], xr, k, op.order_f, acc);
   int64_t p = rot_pix(rep_pixel(r, op.order_c), k, op.order_c);
 #pragma unroll
   for (int j = 0; j < NI; ++j) y[(size_t(row) * Nc + p) * NI + j] = acc[j];
@@ -1375,16 +1476,7 @@ __device__ __forceinline__ void dec_adj_body(const DecOp<T>& op, const T* __rest
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-  int cnt = op.tcnt[q];
-  for (int s = 0; s < cnt; ++s) {
-    size_t at = size_t(s) * op.Rf + q;
-    int64_t ck = rot_pix(op.trow[at], k, op.order_c);
-    T v = op.tval[at];
-    T gv[NI];
-    Load<T>::template vec<NI>(gr + size_t(ck) * NI, gv);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[j] += v * gv[j];
-  }
+  dec_gather_global<T, NI>(op.trow, op.tval, op.Rf, q, op.tcnt[q], gr, k, op.order_c, acc);
   int64_t qk = rot_pix(rep_pixel(q, op.order_f), k, op.order_f);
   size_t o = (size_t(row) * Nf + qk) * NI;
 #pragma unroll
@@ -1549,7 +1641,7 @@ __global__ __launch_bounds__(256) void k_gram_reg(int n, int64_t N, int B, const
 }
 
 // Gram products at the middle levels, K = 4 R + 1 (R = n + 1 = 3..6 branch
-// rows d).  The upper triangle of the K x K Gram is R (R + 1) / 2 blocks of
+// rows d, and 2 with second moments).  The upper triangle of the K x K Gram is R (R + 1) / 2 blocks of
 // 4 x 4 entries between rows a <= b, plus the z column.  Lane class q of a
 // wave owns block (a_q, b_q): its S = 64 / P lanes q S .. q S + S - 1 take S
 // consecutive pixels, load rows a_q, b_q and z there and accumulate the 16
@@ -2492,11 +2584,11 @@ __device__ __forceinline__ void level_item(const LevelTask<T>& t, int64_t bx, in
       dec_fwd_body<T, kL>(t.dec, static_cast<const T*>(t.in0), static_cast<T*>(t.out0), bx, by);
       break;
     case kQConvFwd1:
-      conv_fwd_split_body<T, 1, 8>(t.conv, static_cast<const T*>(t.in0), static_cast<C2*>(t.out0),
+      conv_fwd_split_body<T, 1, kSplitLanes, true>(t.conv, static_cast<const T*>(t.in0), static_cast<C2*>(t.out0),
                                    static_cast<T*>(t.out1), bx, by);
       break;
     case kQConvFwd4:
-      conv_fwd_split_body<T, kL, 8>(t.conv, static_cast<const T*>(t.in0), static_cast<C2*>(t.out0), nullptr, bx,
+      conv_fwd_split_body<T, kL, kSplitLanes, true>(t.conv, static_cast<const T*>(t.in0), static_cast<C2*>(t.out0), nullptr, bx,
                                     by);
       break;
     case kQGram: {
@@ -2536,10 +2628,10 @@ __device__ __forceinline__ void level_item(const LevelTask<T>& t, int64_t bx, in
       break;
     }
     case kQConvAdj1:
-      conv_adj_split_body<T, 1, 8>(t.conv, static_cast<const C2*>(t.in0), static_cast<T*>(t.out0), bx, by);
+      conv_adj_split_body<T, 1, kSplitLanes, true>(t.conv, static_cast<const C2*>(t.in0), static_cast<T*>(t.out0), bx, by);
       break;
     case kQConvAdj4:
-      conv_adj_split_body<T, kL, 8>(t.conv, static_cast<const C2*>(t.in0), static_cast<T*>(t.out0), bx, by);
+      conv_adj_split_body<T, kL, kSplitLanes, true>(t.conv, static_cast<const C2*>(t.in0), static_cast<T*>(t.out0), bx, by);
       break;
     case kQFix1:
       conv_adj_fix_body<T, 1>(t.conv, static_cast<const C2*>(t.in0), static_cast<T*>(t.out0), bx, by);
@@ -2587,6 +2679,8 @@ __global__ __launch_bounds__(256) void k_batch(const LevelTask<T>* __restrict__ 
 }
 
 }  // namespace
+
+int64_t split_blocks(int64_t N) { return (N * kSplitLanes + 255) / 256; }
 
 template <typename T>
 int64_t batch_layout(LevelTask<T>* tasks, int ntasks) {
@@ -2716,10 +2810,9 @@ void launch_conv_fwd(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T
   STL_CHECK(NI == 1 || NI == kL, "conv: unsupported inner width");
   STL_CHECK(conv_fwd_has_variant<T>(NI, variant), "conv: no such variant");
   if (variant == kConvSplit) {
-    constexpr int LP = 8;
-    dim3 grid(nblocks(12 * op.npf * LP, 256), rows);
-    if (NI == 1) k_conv_fwd_split<T, 1, LP><<<grid, 256, 0, s>>>(op, x, y, mod);
-    else k_conv_fwd_split<T, kL, LP><<<grid, 256, 0, s>>>(op, x, y, nullptr);
+    dim3 grid(unsigned(split_blocks(12 * op.npf)), rows);
+    if (NI == 1) k_conv_fwd_split<T, 1, kSplitLanes><<<grid, 256, 0, s>>>(op, x, y, mod);
+    else k_conv_fwd_split<T, kL, kSplitLanes><<<grid, 256, 0, s>>>(op, x, y, nullptr);
     STL_HIP(hipGetLastError());
     return;
   }
@@ -2791,10 +2884,9 @@ bool conv_adj_has_variant(int NI, int variant) {
 template <typename T>
 void conv_adj_gather(const ConvOp<T>& op, int NI, const cplx_t<T>* gy, int rows, T* gx, hipStream_t s, int variant) {
   if (variant == kConvSplit) {
-    constexpr int LP = 8;
-    dim3 grid(nblocks(12 * op.npf * LP, 256), rows);
-    if (NI == 1) k_conv_adj_split<T, 1, LP><<<grid, 256, 0, s>>>(op, gy, gx);
-    else k_conv_adj_split<T, kL, LP><<<grid, 256, 0, s>>>(op, gy, gx);
+    dim3 grid(unsigned(split_blocks(12 * op.npf)), rows);
+    if (NI == 1) k_conv_adj_split<T, 1, kSplitLanes><<<grid, 256, 0, s>>>(op, gy, gx);
+    else k_conv_adj_split<T, kL, kSplitLanes><<<grid, 256, 0, s>>>(op, gy, gx);
     STL_HIP(hipGetLastError());
     return;
   }
@@ -2933,6 +3025,10 @@ void launch_gram(int n, int64_t N, int B, const cplx_t<T>* branch, const cplx_t<
     }                                                                                                      \
     STL_HIP(hipGetLastError());                                                                            \
     return;
+  // K = 9 with moments: the register kernel would hold 135 FP64 sums a thread.
+  if (K == 9 && moments) {
+    switch (2) { STL_GRAM_CLS(2) }
+  }
   switch (n + 1) {
     STL_GRAM_CLS(3) STL_GRAM_CLS(4) STL_GRAM_CLS(5) STL_GRAM_CLS(6)
     default: break;

@@ -44,6 +44,9 @@ void launch_conv_fwd(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T
 template <typename T>
 void launch_conv_adj(const ConvOp<T>& op, int NI, const cplx_t<T>* gy, int rows, T* gx, hipStream_t s,
                      int variant = kConvTiled);
+// 256-thread workgroups (items of a batched launch) of the split convolutions
+// per row of N pixels.
+int64_t split_blocks(int64_t N);
 // Whether the adjoint has this variant for the precision and inner width.
 template <typename T>
 bool conv_adj_has_variant(int NI, int variant);
