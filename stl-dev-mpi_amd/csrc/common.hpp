@@ -120,6 +120,11 @@ constexpr int lds_pitch(int ts, int elem_bytes = 8) {
   return elem_bytes == 8 ? (ts == 32 ? 56 : (ts == 16 ? 40 : 24)) : (ts == 32 ? 44 : (ts == 16 ? 28 : 20));
 }
 
+// Row pitch (in pixels of 4 values) of the windows of the matrix-core forward
+// kernels: the 4 rows of a 4 x 4 pixel block, 16 words each, fall in distinct
+// quarters of the 64 LDS banks when the pitch is 4 or 12 mod 16.
+constexpr int mfma_pitch(int ts) { return ts == 16 ? 28 : 20; }
+
 // Offset (dx, dy) packed as two int8 in an int16.
 __host__ __device__ inline int16_t pack_off(int dx, int dy) {
   return int16_t((dx & 0xFF) | ((dy & 0xFF) << 8));
@@ -160,6 +165,9 @@ struct ConvOp {
   const int32_t* fbo32 = nullptr;  // [R / 64][S]
   const int32_t* fbo16 = nullptr;  // [R / 64][S]
   const int32_t* fbo8 = nullptr;   // [R / 64][S]
+  // The same offsets in the windows of the matrix-core kernels (mfma_pitch).
+  const int32_t* fmo16 = nullptr;  // [R / 64][S]
+  const int32_t* fmo8 = nullptr;   // [R / 64][S]
   const int32_t* tbo32 = nullptr;  // [R / 64][Tn]
   const int32_t* tbo16 = nullptr;  // [R / 64][Tn]
   const int32_t* tbo8 = nullptr;   // [R / 64][Tn]

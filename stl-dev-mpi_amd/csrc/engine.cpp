@@ -1299,20 +1299,50 @@ class EngineT final : public Engine {
           T* gx = NI == 1 ? f_->mg[0].data() : f_->acc[0].data();
           return time_launch([&] { launch_conv_adj<T>(op, NI, gy, rows, gx, s_, v); });
         };
+        // The forward's matrix-core variants replace the others on tiled
+        // levels (FP64: 1.5 to 2 times faster at every size).  In FP32 they
+        // add a row's slots in the same order as the tiled ones but not as
+        // the split one, whose choice is made among the older variants; from
+        // nside 128 on, where it is no candidate, only the older ones that
+        // can still be faster are timed.
+        std::vector<int> more;
+        if (op.tiled && !adj)
+          for (int v = kConvMfma; v < kConvMfma + kFwdMfmas; ++v)
+            if (conv_fwd_mfma_fits(op.order, NI, rows, v)) more.push_back(v);
+        if (!more.empty()) {
+          if (sizeof(T) == 8) cands.clear();
+          else if (op.order > 6) cands = NI == 1 ? std::vector<int>{kConvFaces, kConvFaces32} : std::vector<int>{kConvFaces32};
+        }
         // Two interleaved rounds, each candidate's best: no bias from the
         // order of the candidates or from the first touches of the buffers.
-        std::vector<double> ms(cands.size(), 1e30);
-        for (int round = 0; round < 2; ++round)
-          for (size_t c = 0; c < cands.size(); ++c) ms[c] = std::min(ms[c], timed(cands[c]));
-        double best = ms[0];
+        auto time_all = [&](const std::vector<int>& vs) {
+          std::vector<double> ms(vs.size(), 1e30);
+          for (int round = 0; round < 2; ++round)
+            for (size_t c = 0; c < vs.size(); ++c) ms[c] = std::min(ms[c], timed(vs[c]));
+          for (size_t c = 0; c < vs.size(); ++c) tune_ms_.push_back(TuneRecord{n, kind, vs[c], ms[c]});
+          return ms;
+        };
         int pick = kConvTiled;
-        for (size_t c = 1; c < cands.size(); ++c)
-          if (ms[c] < 0.97 * ms[0] && ms[c] < best) {
-            best = ms[c];
-            pick = cands[c];
-          }
+        double best = 1e30;
+        if (!cands.empty()) {
+          const std::vector<double> ms = time_all(cands);
+          best = ms[0];
+          pick = cands[0];
+          for (size_t c = 1; c < cands.size(); ++c)
+            if (ms[c] < 0.97 * ms[0] && ms[c] < best) {
+              best = ms[c];
+              pick = cands[c];
+            }
+        }
+        if (!more.empty() && pick != kConvSplit) {
+          const std::vector<double> ms = time_all(more);
+          for (size_t c = 0; c < more.size(); ++c)
+            if (ms[c] < best) {
+              best = ms[c];
+              pick = more[c];
+            }
+        }
         conv_var_[n][kind] = pick;
-        for (size_t c = 0; c < cands.size(); ++c) tune_ms_.push_back(TuneRecord{n, kind, cands[c], ms[c]});
         std::lock_guard<std::mutex> lock(tune_mutex());
         tune_cache()[key] = pick;
       }

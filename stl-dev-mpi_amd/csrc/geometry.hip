@@ -765,12 +765,12 @@ __global__ void k_lin_off32(int64_t n, const int32_t* __restrict__ off, int pitc
 
 // Re-slots (cnt, ids, off, coef) of Sn slots over R rows into union slots
 // (capacity a multiple of 4: the tiled loops run whole chunks of 4 slots);
-// returns the new capacity.  bcnt: the blocks' counts; lin[i]: the blocks'
-// offsets in linear form for window pitches pitch[i].
+// returns the new capacity.  bcnt: the blocks' counts; lin: the blocks' offsets
+// in linear form for each window pitch.
 template <typename T, bool kTrans>
 int union_slots(int64_t R, int Sn, DevArray<uint8_t>& cnt, DevArray<int32_t>& ids, DevArray<int16_t>& off,
-                DevArray<T>& coef, DevArray<int32_t>& bcnt, const int (&pitch)[3], DevArray<int32_t>* const (&lin)[3],
-                hipStream_t s) {
+                DevArray<T>& coef, DevArray<int32_t>& bcnt,
+                const std::vector<std::pair<int, DevArray<int32_t>*>>& lin, hipStream_t s) {
   STL_CHECK(R % 64 == 0, "union slots: blocks of 64 rows");
   const int64_t nb = R / 64;
   bcnt.resize(size_t(nb));
@@ -789,10 +789,10 @@ int union_slots(int64_t R, int Sn, DevArray<uint8_t>& cnt, DevArray<int32_t>& id
                                                        bcnt.data(), boff.data(), ucnt.data(), uids.data(),
                                                        uoff.data(), ucoef.data());
   STL_HIP(hipGetLastError());
-  for (int i = 0; i < 3; ++i) {
-    lin[i]->resize(boff.size());
-    k_lin_off32<<<blocks_for(int64_t(boff.size()), 256), 256, 0, s>>>(int64_t(boff.size()), boff.data(), pitch[i],
-                                                                     lin[i]->data());
+  for (const auto& [pitch, out] : lin) {
+    out->resize(boff.size());
+    k_lin_off32<<<blocks_for(int64_t(boff.size()), 256), 256, 0, s>>>(int64_t(boff.size()), boff.data(), pitch,
+                                                                     out->data());
     STL_HIP(hipGetLastError());
   }
   STL_HIP(hipStreamSynchronize(s));
@@ -820,13 +820,19 @@ void mirror_store(int order, ConvStore<T>& st, hipStream_t s) {
   st.slots = host_sum_u8(st.cnt);
   st.tslots = host_sum_u8(st.tcnt);
   if (st.tiled) {
-    // Forward windows: pitch SW = TS + 2 kWin; the adjoints': lds_pitch(TS)
-    // of their complex elements.
+    // Forward windows: pitch SW = TS + 2 kWin, or mfma_pitch(TS); the
+    // adjoints': lds_pitch(TS) of their complex elements.
     st.S = union_slots<T, false>(R2, st.S, st.cnt, st.cell, st.off, st.coef, st.fbcnt,
-                                 {32 + 2 * kWin, 16 + 2 * kWin, 8 + 2 * kWin}, {&st.fbo32, &st.fbo16, &st.fbo8}, s);
-    st.Tn = union_slots<T, true>(R2, st.Tn, st.tcnt, st.trow, st.toff, st.tcoef, st.tbcnt,
-                                 {lds_pitch(32, 2 * sizeof(T)), lds_pitch(16, 2 * sizeof(T)), lds_pitch(8, 2 * sizeof(T))},
-                                 {&st.tbo32, &st.tbo16, &st.tbo8}, s);
+                                 {{32 + 2 * kWin, &st.fbo32},
+                                  {16 + 2 * kWin, &st.fbo16},
+                                  {8 + 2 * kWin, &st.fbo8},
+                                  {mfma_pitch(16), &st.fmo16},
+                                  {mfma_pitch(8), &st.fmo8}},
+                                 s);
+    constexpr int cb = 2 * sizeof(T);
+    st.Tn = union_slots<T, true>(
+        R2, st.Tn, st.tcnt, st.trow, st.toff, st.tcoef, st.tbcnt,
+        {{lds_pitch(32, cb), &st.tbo32}, {lds_pitch(16, cb), &st.tbo16}, {lds_pitch(8, cb), &st.tbo8}}, s);
   }
 }
 

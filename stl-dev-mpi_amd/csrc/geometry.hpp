@@ -22,7 +22,7 @@ struct ConvStore {
   DevArray<int32_t> cell, trow;
   DevArray<int16_t> off, toff;
   DevArray<T> coef, tcoef;
-  DevArray<int32_t> fbcnt, fbo32, fbo16, fbo8;  // ConvOp::fbcnt / fbo* (tiled levels)
+  DevArray<int32_t> fbcnt, fbo32, fbo16, fbo8, fmo16, fmo8;  // ConvOp::fbcnt / fbo* / fmo* (tiled levels)
   DevArray<int32_t> tbcnt, tbo32, tbo16, tbo8;  // ConvOp::tbcnt / tbo* (tiled levels)
   // Entries stored (forward and transposed), without the union slots' zeros.
   double slots = 0.0, tslots = 0.0;
@@ -41,6 +41,7 @@ struct ConvStore {
     v.cnt = cnt.data(); v.cell = cell.data(); v.off = off.data(); v.coef = coef.data();
     v.tcnt = tcnt.data(); v.trow = trow.data(); v.toff = toff.data(); v.tcoef = tcoef.data();
     v.fbcnt = fbcnt.data(); v.fbo32 = fbo32.data(); v.fbo16 = fbo16.data(); v.fbo8 = fbo8.data();
+    v.fmo16 = fmo16.data(); v.fmo8 = fmo8.data();
     v.tbcnt = tbcnt.data(); v.tbo32 = tbo32.data(); v.tbo16 = tbo16.data(); v.tbo8 = tbo8.data();
     v.nfix = nfix;
     v.fix_cell = fix_cell.data(); v.fix_ptr = fix_ptr.data(); v.fix_row = fix_row.data();
@@ -49,7 +50,8 @@ struct ConvStore {
   }
   size_t bytes() const {
     return cnt.bytes() + tcnt.bytes() + cell.bytes() + trow.bytes() + off.bytes() + toff.bytes() + coef.bytes() +
-           tcoef.bytes() + fbcnt.bytes() + fbo32.bytes() + fbo16.bytes() + fbo8.bytes() + tbcnt.bytes() + tbo32.bytes() +
+           tcoef.bytes() + fbcnt.bytes() + fbo32.bytes() + fbo16.bytes() + fbo8.bytes() + fmo16.bytes() +
+           fmo8.bytes() + tbcnt.bytes() + tbo32.bytes() +
            tbo16.bytes() + tbo8.bytes() + fix_cell.bytes() + fix_ptr.bytes() + fix_row.bytes() +
            fix_coef.bytes();
   }

@@ -607,6 +607,12 @@ __device__ inline BlockSlots fwd_block_slots(const ConvOp<T>& op, int fr, int64_
   const int32_t* lin = TS == 32 ? op.fbo32 : (TS == 16 ? op.fbo16 : op.fbo8);
   return BlockSlots{lin + blk * op.S, op.fbcnt[blk]};
 }
+// Forward slots in the windows of the matrix-core kernels.
+template <int TS, typename T>
+__device__ inline BlockSlots mfma_block_slots(const ConvOp<T>& op, int fr, int64_t base, int rl) {
+  const int64_t blk = wave_block(op.npf, fr, base, rl);
+  return BlockSlots{(TS == 16 ? op.fmo16 : op.fmo8) + blk * op.S, op.fbcnt[blk]};
+}
 
 // A 32 x 32 tile is a 16-wave workgroup: two of them per CU need 8 waves per
 // SIMD, i.e. at most 64 VGPRs; at 7 waves only one fits.
@@ -909,6 +915,256 @@ __device__ __forceinline__ void pipelined_slots(const int32_t* __restrict__ off,
     run(a1, (c + 1) * U);
   }
   if (c < nch) run(a0, c * U);
+}
+
+// ---------------------------------------------------------------------------
+// Forward convolution on the matrix cores (TS x TS tiles).  A rep pixel's
+// coefficients of one slot (4 gauges, re or im) are a column, its inputs there
+// (the 4 orientations of a modulus, or the 4 rotated faces of a map) a row,
+// and the 4 x 4 products of 16 pixels (FP32: K = 1, one slot) or of 4 pixels
+// (FP64: K = 4 slots) are one instruction.  What bounds the convolution is the
+// coefficient stream, 32 (FP32) or 64 (FP64) bytes a slot and pixel: a lane
+// holds one gauge's coefficient and one accumulator column, a quarter of the
+// registers of a thread per pixel, so a workgroup keeps FW faces x RW rows of
+// sums and each coefficient is loaded once for all of them.
+// FP32: slot by slot with one rounding per product and sum, the bits of the
+// thread-per-pixel kernels.
+// Measured against the thread-per-pixel kernels (us): FP64 branches of one
+// nside-1024 map, levels 0, 1, 2: 2710, 1423, 561 -> 1872, 802, 312; of 4 maps
+// at nside 128, level 0: 216 -> 112; of one map at nside 64: 30 -> 14.5 (its
+// z: 22 -> 9.5).  FP32 branches of two nside-512 maps: 619 -> 435; of one
+// nside-1024 map, level 0: 1200 -> 1047 (its z stays with the thread-per-pixel
+// form, 765 against 843).  FP64 stays on 8 x 8 tiles at most sizes: their
+// windows' halo is read from the L2, and 3 workgroups fit a CU.
+// ---------------------------------------------------------------------------
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+
+// Windows of FW faces (kind k = fg FW + f) and RW rows, [row][face][pos][4
+// orientations] (NI = 4), or [row][pos][4 faces] (NI = 1).  The pixel of face
+// shift 0 at a position gives the other faces' by rotation.
+template <typename T, int NI, int TS, int FW, int RW, int NT>
+__device__ __forceinline__ void stage_rows(const ConvOp<T>& op, const T* __restrict__ x, int rows, int row0, int fr,
+                                           int fg, bool m, int x0, int y0, T* xs) {
+  constexpr int SW = TS + 2 * kWin, PW = mfma_pitch(TS), SA = SW * PW;
+  const bool inside = window_inside<TS>(x0, y0, op.order);
+  const int64_t N = 12 * op.npf;
+  for (int idx = threadIdx.x; idx < SW * SW; idx += NT) {
+    const int pi = stage_index<SW>(m, idx);
+    const int wx = pi % SW, wy = pi / SW, at = (wy * PW + wx) * 4;
+    const int64_t p0 = window_pixel(inside, 4 * fr, m, x0 - kWin + wx, y0 - kWin + wy, op.order);
+    T v[RW][FW][NI];
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int f = 0; f < FW; ++f) {
+        const int64_t p = rot_pix(p0 >= 0 ? p0 : 0, fg * FW + f, op.order);
+        Load<T>::template vec<NI>(x + (size_t(min(row0 + r, rows - 1)) * N + p) * NI, v[r][f]);
+      }
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int f = 0; f < FW; ++f)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          xs[NI == 1 ? r * SA * 4 + at + f : (r * FW + f) * SA * 4 + at + j] = p0 >= 0 ? v[r][f][j] : T(0);
+  }
+}
+
+// Tile unit, face group and first row of a workgroup.
+template <int TS, int FW, int RW>
+struct MfmaTile {
+  int fr, fg, row0, x0, y0;
+  bool m;
+  int64_t base;
+  __device__ MfmaTile(int order, int64_t npf, int rows) {
+    int64_t tr, tile;
+    int rg;
+    tile_group<TS, FW>(order, (rows + RW - 1) / RW, tr, fg, rg);
+    unit_tile(tr, npf / (TS * TS), fr, tile, m);
+    base = tile * (TS * TS);
+    row0 = rg * RW;
+    x0 = int(compress_bits(uint32_t(base)));
+    y0 = int(compress_bits(uint32_t(base >> 1)));
+  }
+};
+
+// One output: gauge i of the rep row's sums at a pixel of face shift k, as
+// gauge g of that face.
+template <typename T>
+__device__ __forceinline__ cplx_t<T> face_value(T re, T im, int k, int g, bool m) {
+  return make_c<T>(re, gauge_conj(k, g) != m ? -im : im);
+}
+
+template <int NI, int TS, int FW, int RW, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void k_conv_fwd_mfma32(ConvOp<float> op, const float* __restrict__ x,
+                                                                int rows, float2* __restrict__ y,
+                                                                float* __restrict__ mod) {
+  constexpr int SW = TS + 2 * kWin, PW = mfma_pitch(TS), SA = SW * PW;
+  constexpr int NF = NI == 1 ? 1 : FW;          // windows per row
+  constexpr int GW = TS * TS / 16 / WAVES;      // 4 x 4 pixel blocks per wave
+  static_assert(GW == 1 || GW == 2 || GW == 4, "the wave's blocks share an 8 x 8 block's offsets");
+  __shared__ float xs[RW * NF * SA * 4];
+  const MfmaTile<TS, FW, RW> t(op.order, op.npf, rows);
+  stage_rows<float, NI, TS, FW, RW, WAVES * 64>(op, x, rows, t.row0, t.fr, t.fg, t.m, t.x0, t.y0, xs);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, jj = lane & 3;
+  const int rl = wave * GW * 16 + (lane >> 2);  // rep pixel of block 0
+  const int pos = (int(compress_bits(uint32_t(rl >> 1))) + kWin) * PW + int(compress_bits(uint32_t(rl))) + kWin;
+  const float* win = xs + pos * 4 + jj;
+  const uint32_t co = uint32_t((int64_t(t.fr) * op.npf + t.base + rl) * 32 + jj * 8);
+  const BlockSlots bs = mfma_block_slots<TS>(op, t.fr, t.base, rl);
+  mfma_f4 re[GW][RW][NF], im[GW][RW][NF];
+#pragma unroll
+  for (int w = 0; w < GW; ++w)
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) re[w][r][f] = im[w][r][f] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+  const float2* coef = reinterpret_cast<const float2*>(op.coef);
+  pipelined_slots<4, GW, float2>(
+      bs.off, bs.cnt, op.S,
+      [&](int s0, int u, int w) {
+        return plane_load(coef + (size_t(s0) * op.R + size_t(u) * op.R + size_t(w) * 16) * 4, co);
+      },
+      [&](int32_t o, const float2(&a)[GW]) {
+#pragma unroll
+        for (int w = 0; w < GW; ++w)
+#pragma unroll
+          for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+              const float b = win[((r * NF + f) * SA + o + (w & 1) * 4 + (w >> 1) * 4 * PW) * 4];
+              re[w][r][f] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[w].x, b, re[w][r][f], 0, 0, 0);
+              im[w][r][f] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[w].y, b, im[w][r][f], 0, 0, 0);
+            }
+      });
+  const int64_t N = 12 * op.npf;
+#pragma unroll
+  for (int w = 0; w < GW; ++w) {
+    const int li = rep_lane<TS>(t.m, rl + w * 16);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const int row = t.row0 + r;
+      if (row >= rows) break;
+      if constexpr (NI == 1) {
+        // Lane column = face shift: gauge g of an odd shift is rep gauge g ^ 2.
+        const int64_t p = tile_out<TS>(4 * t.fr + jj, t.m, t.base, op.order) + li;
+        float2 v[kL];
+        float h[kL];
+#pragma unroll
+        for (int g = 0; g < kL; ++g) {
+          v[g] = face_value<float>(jj & 1 ? re[w][r][0][g ^ 2] : re[w][r][0][g],
+                                   jj & 1 ? im[w][r][0][g ^ 2] : im[w][r][0][g], jj, g, t.m);
+          y[(size_t(row) * kL + g) * N + p] = v[g];
+          h[g] = hypot(v[g].x, v[g].y);
+        }
+        if (mod != nullptr)
+          *reinterpret_cast<float4*>(mod + (size_t(row) * N + p) * kL) = make_float4(h[0], h[1], h[2], h[3]);
+      } else {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const int k = FW == 4 ? f : t.fg * FW + f;
+          const int64_t p = tile_out<TS>(4 * t.fr + k, t.m, t.base, op.order) + li;
+#pragma unroll
+          for (int g = 0; g < kL; ++g)
+            y[((size_t(row) * kL + g) * N + p) * NI + jj] =
+                face_value<float>(k & 1 ? re[w][r][f][g ^ 2] : re[w][r][f][g],
+                                  k & 1 ? im[w][r][f][g ^ 2] : im[w][r][f][g], k, g, t.m);
+        }
+      }
+    }
+  }
+}
+
+// FP64: lane (i = l & 3, b = l >> 2 & 3, k = l >> 4) loads gauge i of pixel b
+// at slot k of a chunk of 4, and the column of the same i at that slot; its
+// result is the sum of gauge l >> 4 of pixel b, column i.
+template <int NI, int TS, int FW, int RW, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void k_conv_fwd_mfma64(ConvOp<double> op, const double* __restrict__ x,
+                                                                int rows, double2* __restrict__ y,
+                                                                double* __restrict__ mod) {
+  constexpr int SW = TS + 2 * kWin, PW = mfma_pitch(TS), SA = SW * PW;
+  constexpr int NF = NI == 1 ? 1 : FW;
+  constexpr int Q = TS * TS / 4 / WAVES;  // 2 x 2 pixel blocks per wave
+  static_assert(Q == 2 || Q == 4 || Q == 8 || Q == 16, "the wave's blocks share an 8 x 8 block's offsets");
+  __shared__ double xs[RW * NF * SA * 4];
+  const MfmaTile<TS, FW, RW> t(op.order, op.npf, rows);
+  stage_rows<double, NI, TS, FW, RW, WAVES * 64>(op, x, rows, t.row0, t.fr, t.fg, t.m, t.x0, t.y0, xs);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = lane & 3, b = (lane >> 2) & 3, k4 = lane >> 4;
+  const int rl = wave * Q * 4 + b;  // rep pixel of block 0
+  const int pos = (int(compress_bits(uint32_t(rl >> 1))) + kWin) * PW + int(compress_bits(uint32_t(rl))) + kWin;
+  const double* win = xs + pos * 4 + i;
+  const BlockSlots bs = mfma_block_slots<TS>(op, t.fr, t.base, rl);
+  const int32_t* off = bs.off + k4;
+  const double2* cp = reinterpret_cast<const double2*>(op.coef) +
+                      (size_t(k4) * op.R + size_t(int64_t(t.fr) * op.npf + t.base + rl)) * kL + i;
+  const size_t step = size_t(op.R) * 4 * kL;
+  double re[Q][RW][NF], im[Q][RW][NF];
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) re[q][r][f] = im[q][r][f] = 0.0;
+  double2 a0[Q], a1[Q];
+  int32_t o0, o1;
+  // Unconditional, the last chunk of the capacity again past the count (as in pipelined_slots).
+  auto fetch = [&](double2(&a)[Q], int32_t& o, int c) {
+    const int cc = min(c, op.S / 4 - 1);
+    const double2* p = cp + size_t(cc) * step;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) a[q] = p[q * 4 * kL];
+    o = off[cc * 4];
+  };
+  auto run = [&](const double2(&a)[Q], int32_t o) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int r = 0; r < RW; ++r)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          // Block q at NESTED offset 4 q: its position in the 8 x 8 block.
+          constexpr int kX[16] = {0, 2, 0, 2, 4, 6, 4, 6, 0, 2, 0, 2, 4, 6, 4, 6};
+          constexpr int kY[16] = {0, 0, 2, 2, 0, 0, 2, 2, 4, 4, 6, 6, 4, 4, 6, 6};
+          const double v = win[((r * NF + f) * SA + o + kX[q] + kY[q] * PW) * 4];
+          re[q][r][f] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[q].x, v, re[q][r][f], 0, 0, 0);
+          im[q][r][f] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[q].y, v, im[q][r][f], 0, 0, 0);
+        }
+  };
+  const int nch = (bs.cnt + 3) / 4;
+  if (nch > 0) {
+    fetch(a0, o0, 0);
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {
+      fetch(a1, o1, c + 1);
+      run(a0, o0);
+      fetch(a0, o0, c + 2);
+      run(a1, o1);
+    }
+    if (c < nch) run(a0, o0);
+  }
+  const int64_t N = 12 * op.npf;
+  // This lane's result: rep gauge k4 of pixel b, column i.
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int li = rep_lane<TS>(t.m, rl + q * 4);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const int row = t.row0 + r;
+      if (row >= rows) break;
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const int k = NI == 1 ? i : (FW == 4 ? f : t.fg * FW + f);
+        const int g = gauge_src(k, k4);
+        const int64_t p = tile_out<TS>(4 * t.fr + k, t.m, t.base, op.order) + li;
+        const double2 v = face_value<double>(re[q][r][f], im[q][r][f], k, g, t.m);
+        y[((size_t(row) * kL + g) * N + p) * NI + (NI == 1 ? 0 : i)] = v;
+        if (NI == 1 && mod != nullptr) mod[(size_t(row) * N + p) * kL + g] = hypot(v.x, v.y);
+      }
+    }
+  }
 }
 
 // Window positions staged per batch by the adjoints (every load of a batch
@@ -2798,10 +3054,53 @@ void conv_fwd_faces32(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<
   }
 }
 
+// Matrix-core forward: variant kConvMfma + i of the table below (TS, FW, RW,
+// waves); the rows are taken RW at a time, the last group's missing rows
+// repeat its last one.
+template <typename T, int NI, int TS, int FW, int RW, int WAVES>
+void conv_fwd_mfma(const ConvOp<T>& op, const T* x, int rows, cplx_t<T>* y, T* mod, hipStream_t s) {
+  constexpr int ways = NI == 1 ? 1 : 4 / FW;
+  const dim3 grid(unsigned(3 * op.npf / (TS * TS) * ways * ((rows + RW - 1) / RW)));
+  constexpr int FS = NI == 1 ? 4 : FW;
+  if constexpr (sizeof(T) == 4) k_conv_fwd_mfma32<NI, TS, FS, RW, WAVES><<<grid, WAVES * 64, 0, s>>>(op, x, rows, y, mod);
+  else k_conv_fwd_mfma64<NI, TS, FS, RW, WAVES><<<grid, WAVES * 64, 0, s>>>(op, x, rows, y, mod);
+}
+
+template <typename T>
+void conv_fwd_mfma_variant(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T>* y, T* mod, int i,
+                           hipStream_t s) {
+  constexpr bool F = sizeof(T) == 4;
+  if (NI == 1) {
+    switch (i) {
+      case 0: conv_fwd_mfma<T, 1, 8, 4, 1, 4>(op, x, rows, y, mod, s); break;
+      case 1: conv_fwd_mfma<T, 1, 8, 4, 2, 4>(op, x, rows, y, mod, s); break;
+      case 2: conv_fwd_mfma<T, 1, 16, 4, 1, 4>(op, x, rows, y, mod, s); break;
+      default: conv_fwd_mfma<T, 1, 16, 4, 2, 8>(op, x, rows, y, mod, s); break;
+    }
+  } else {
+    switch (i) {
+      case 0: conv_fwd_mfma<T, kL, 8, 4, 1, 4>(op, x, rows, y, nullptr, s); break;
+      case 2: conv_fwd_mfma<T, kL, 16, F ? 4 : 2, 1, 8>(op, x, rows, y, nullptr, s); break;
+      default: conv_fwd_mfma<T, kL, 16, F ? 4 : 2, 2, 16>(op, x, rows, y, nullptr, s); break;
+    }
+  }
+}
+
 template <typename T>
 bool conv_fwd_has_variant(int NI, int variant) {
   if (variant == kConvFaces32) return NI == 1 || sizeof(T) == 4;
-  return variant >= kConvTiled && variant < kConvFaces32;
+  return variant >= kConvTiled && variant < kConvMfma + kFwdMfmas;
+}
+
+// Tiles of 8 x 8 (variants 0, 1) or 16 x 16 (2, 3) pixels fit the face; the
+// byte offset of a row's coefficients within a slot is 32 bits wide (nside <=
+// 4096); two rows per workgroup (1, 3) need two rows, and on 8 x 8 tiles they
+// pay for the maps only (the modulus windows of two rows leave one workgroup
+// of 4 waves per CU: 260 against 215 us at 2 rows of nside 512 in FP32).
+bool conv_fwd_mfma_fits(int order, int NI, int rows, int variant) {
+  const int i = variant - kConvMfma;
+  if (order > 12 || order < (i < 2 ? 3 : 4)) return false;
+  return i % 2 == 0 || (rows >= 2 && !(i == 1 && NI != 1));
 }
 
 template <typename T>
@@ -2809,6 +3108,8 @@ void launch_conv_fwd(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T
                      int variant) {
   STL_CHECK(NI == 1 || NI == kL, "conv: unsupported inner width");
   STL_CHECK(conv_fwd_has_variant<T>(NI, variant), "conv: no such variant");
+  STL_CHECK(variant < kConvMfma || (op.tiled && conv_fwd_mfma_fits(op.order, NI, rows, variant)),
+            "conv: no such variant");
   if (variant == kConvSplit) {
     dim3 grid(unsigned(split_blocks(12 * op.npf)), rows);
     if (NI == 1) k_conv_fwd_split<T, 1, kSplitLanes><<<grid, 256, 0, s>>>(op, x, y, mod);
@@ -2818,7 +3119,8 @@ void launch_conv_fwd(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T
   }
   if (op.tiled) {
     const int TS = op.order >= 4 ? 16 : 8;
-    if (variant == kConvTiled32 && op.order >= 5) conv_fwd_tiled<T, 32>(op, NI, x, rows, y, mod, s);
+    if (variant >= kConvMfma) conv_fwd_mfma_variant<T>(op, NI, x, rows, y, mod, variant - kConvMfma, s);
+    else if (variant == kConvTiled32 && op.order >= 5) conv_fwd_tiled<T, 32>(op, NI, x, rows, y, mod, s);
     else if (variant == kConvFaces32 && op.order >= 5) conv_fwd_faces32<T>(op, NI, x, rows, y, mod, s);
     else if (variant == kConvFaces && TS == 16) conv_fwd_faces<T, 16>(op, NI, x, rows, y, mod, s);
     else if (variant == kConvFaces) conv_fwd_faces<T, 8>(op, NI, x, rows, y, mod, s);

@@ -38,6 +38,11 @@ using cplx_t = typename Complex2<T>::type;
 // or several rotated faces per workgroup on 32 x 32 tiles.
 constexpr int kConvTiled = 0, kConvFaces = 1, kConvTiled8 = 2, kConvTiled32 = 3, kConvSplit = 4,
               kConvFaces32 = 5;
+// Matrix-core forward variants kConvMfma .. kConvMfma + kFwdMfmas - 1: 8 x 8
+// tiles with 1 or 2 rows per workgroup, 16 x 16 tiles with 1 or 2; whether one
+// serves `rows` rows of inner width NI.
+constexpr int kConvMfma = 6, kFwdMfmas = 4;
+bool conv_fwd_mfma_fits(int order, int NI, int rows, int variant);
 template <typename T>
 void launch_conv_fwd(const ConvOp<T>& op, int NI, const T* x, int rows, cplx_t<T>* y, T* modulus_out,
                      hipStream_t s, int variant = kConvTiled);

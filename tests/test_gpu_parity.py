@@ -458,3 +458,27 @@ def test_batched_levels_agree_with_level_launches(precision):
     else:
         assert max(family_errors(got[0], ref0[0], plan).values()) < 1e-6
         assert rel(got[2], ref0[2]) < 1e-5
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nside,J,batch", [(8, 1, 1), (16, 1, 3), (32, 2, 2), (64, 2, 5), (128, 3, 1)])
+def test_matrix_core_forward_agrees_with_the_tiled_one(nside, J, batch, precision):
+    """The timed choice of forward convolutions (the matrix-core forms on tiled levels: 8 x 8 and 16 x 16
+    tiles, one or two rows per workgroup, odd row counts among them) against the 16 x 16 thread-per-pixel
+    form: the same bits in FP32, where both add a row's slots in the same order (a level whose choice is
+    the 8-lane split form is held to rounding), FP64 to rounding."""
+    from stl_port import NativeEngine
+    x = np.random.default_rng(nside + batch).standard_normal((batch, 12 * nside * nside))
+    out = []
+    for v in (0, None):
+        print(f"[gpu] forward nside={nside} J={J} B={batch} {precision} variant={v}", flush=True)
+        with NativeEngine(nside, J, batch=batch, precision=precision, conv_variant=v, batch_nside=0) as e:
+            out.append((e.forward(x)[0], e.info()["conv_variants"]))
+    (v0, _), (v1, kinds) = out
+    if precision == "fp64":
+        assert all(k >= 6 for level in kinds for k in level[:2])  # the matrix-core forms
+    if precision == "mixed" and not any(k == 4 for level in kinds for k in level[:2]):
+        assert np.array_equal(v0, v1)
+    # Rounding of 50 slots' sums, twice (z and its modulus' wavelets), a product and J levels.
+    eps = (2.0 ** -24 if precision == "mixed" else 2.0 ** -53) * 50 * 4 * (J + 1)
+    assert np.abs(v1 - v0).max() <= eps * np.abs(v0).max()
