@@ -295,17 +295,18 @@ class EngineT final : public Engine {
     std::vector<DevArray<T>> maps, M;
     std::vector<DevArray<C2>> z, br;
     // Reverse buffers: gbr / gzp / acc[0] hold level 0, gbr1 / gzp1 / acc[1]
-    // level 1, gbr2 / gzp2 and acc[2 + (n & 1)] the levels n >= 2, so that
-    // level 0's and level 1's gV and branch adjoints can run beside the
-    // coarser levels' reverse.
-    DevArray<C2> gbr, gzp, gz, gbr1, gzp1, gbr2, gzp2;
-    DevArray<T> acc[4], mg[2];
-    // Reverse buffers of every batched level (from level qc on), so that one
-    // launch can hold a step of all of them: gV, z part, chain, gz and map
-    // cotangent.
+    // level 1, lgbr / lgzp / lchain the levels n >= 2 (each its own), so that
+    // every level's gV and branch adjoint can run beside the coarser levels'
+    // reverse.
+    DevArray<C2> gbr, gzp, gz, gbr1, gzp1;
+    std::vector<DevArray<C2>> lgbr, lgzp;
+    DevArray<T> acc[2], mg[2];
+    std::vector<DevArray<T>> lchain;
+    // gz and map cotangent of every batched level (from level qc on), so that
+    // one launch can hold a step of all of them.
     int qc = 0;
-    std::vector<DevArray<C2>> qgbr, qgzp, qgz;
-    std::vector<DevArray<T>> qchain, qmg;
+    std::vector<DevArray<C2>> qgz;
+    std::vector<DevArray<T>> qmg;
   };
 
  public:
@@ -566,25 +567,19 @@ class EngineT final : public Engine {
     }
   }
 
-  // Reverse buffers of level n (levels 0 and 1 apart from the others).
-  // Level-n buffers.  Keep store: z and branches of every level; the reverse
-  // buffers of levels 0 and 1 apart from the others.  Recompute store: one
-  // level's z, branches and reverse buffers at a time.
+  // Level-n buffers.  Keep store: z, branches and reverse buffers of every
+  // level.  Recompute store: one level's at a time.
   C2* z_of(int n) { return f_->z[f_->recompute ? 0 : n].data(); }
   C2* br_of(int n) { return f_->br[f_->recompute ? 0 : n].data(); }
-  // The batched levels (n >= qc_) have reverse buffers of their own.
   bool batched(int n) const { return n >= qc_ && batch_on(); }
   C2* gbr_of(int n) {
-    if (batched(n)) return f_->qgbr[n].data();
-    return n == 0 || f_->recompute ? f_->gbr.data() : n == 1 ? f_->gbr1.data() : f_->gbr2.data();
+    return n == 0 || f_->recompute ? f_->gbr.data() : n == 1 ? f_->gbr1.data() : f_->lgbr[n].data();
   }
   C2* gzp_of(int n) {
-    if (batched(n)) return f_->qgzp[n].data();
-    return n == 0 || f_->recompute ? f_->gzp.data() : n == 1 ? f_->gzp1.data() : f_->gzp2.data();
+    return n == 0 || f_->recompute ? f_->gzp.data() : n == 1 ? f_->gzp1.data() : f_->lgzp[n].data();
   }
   T* chain_of(int n) {
-    if (batched(n)) return f_->qchain[n].data();
-    return f_->acc[f_->recompute ? (n & 1) : n < 2 ? n : 2 + (n & 1)].data();
+    return f_->recompute ? f_->acc[n & 1].data() : n < 2 ? f_->acc[n].data() : f_->lchain[n].data();
   }
   C2* gz_of(int n) { return batched(n) ? f_->qgz[n].data() : f_->gz.data(); }
   T* mg_of(int n) { return batched(n) ? f_->qmg[n].data() : f_->mg[n % 2].data(); }
@@ -827,25 +822,19 @@ class EngineT final : public Engine {
       f_->gzp1.resize(f_->z[1].size());
       f_->acc[1].resize(f_->M[1].size());
     }
-    if (levels_ > 2) {
-      size_t g2 = 0;
-      for (int n = 2; n < levels_; ++n) g2 = std::max(g2, f_->br[n].size());
-      f_->gbr2.resize(g2);
-      f_->gzp2.resize(f_->z[2].size());
-      f_->acc[2].resize(f_->M[2].size());
-      f_->acc[3].resize(f_->M[2].size());
+    f_->lgbr.resize(levels_);
+    f_->lgzp.resize(levels_);
+    f_->lchain.resize(levels_);
+    for (int n = 2; n < levels_; ++n) {
+      f_->lgbr[n].resize(f_->br[n].size());
+      f_->lgzp[n].resize(f_->z[n].size());
+      f_->lchain[n].resize(f_->M[n].size());
     }
     f_->qc = qc_;
-    f_->qgbr.resize(levels_);
-    f_->qgzp.resize(levels_);
     f_->qgz.resize(levels_);
-    f_->qchain.resize(levels_);
     f_->qmg.resize(levels_);
     for (int n = qc_; n < levels_; ++n) {
-      f_->qgbr[n].resize(f_->br[n].size());
-      f_->qgzp[n].resize(f_->z[n].size());
       f_->qgz[n].resize(f_->z[n].size());
-      f_->qchain[n].resize(f_->M[n].size());
       f_->qmg[n].resize(f_->maps[n].size());
     }
     f_->bytes = device_bytes_live() - live0;
@@ -857,14 +846,12 @@ class EngineT final : public Engine {
     auto len = [&](int n) { return n < levels_ ? size_t(N_[n]) : size_t(0); };
     size_t e = 0, c = 0;  // real and complex elements
     for (int n = 0; n < levels_; ++n) {
-      e += size_t(B_) * len(n) * (1 + (n + 1) * kL);
-      c += size_t(B_) * len(n) * kL * (1 + (n + 1) * kL);
+      // maps, moduli and the chain; z, branches and their cotangents
+      e += size_t(B_) * len(n) * (1 + 2 * (n + 1) * kL);
+      c += size_t(B_) * len(n) * 2 * kL * (1 + (n + 1) * kL);
     }
-    size_t br2 = 0;
-    for (int n = 2; n < levels_; ++n) br2 = std::max(br2, size_t(n + 1) * B_ * kL * len(n) * kL);
-    c += size_t(B_) * kL * kL * len(0) + 2 * size_t(B_) * kL * len(0) + 2 * size_t(B_) * kL * kL * len(1) +
-         size_t(B_) * kL * len(1) + br2 + size_t(B_) * kL * len(2);
-    e += size_t(B_) * kL * (len(0) + 2 * len(1) + 6 * len(2)) + 2 * size_t(B_) * len(0);
+    c += size_t(B_) * kL * len(0);  // gz
+    e += 2 * size_t(B_) * len(0);   // mg
     return e * sizeof(T) + c * sizeof(C2);
   }
 
@@ -1059,20 +1046,21 @@ class EngineT final : public Engine {
     else
       launch_gram<T>(n, N, B_, br_of(n), z_of(n), moments, nb, gpart_[n].data(), gpart2_[n].data(),
                      zpart_[n].data(), mv, s_);
-    launch_reduce_parts(gpart_[n].data(), nb, m * 2, gsum_[n].data(), s_);
-    if (moments) launch_reduce_parts(gpart2_[n].data(), nb, m, gsum2_[n].data(), s_);
     prof_.stop(id, tag("gram", n), double(rows) * kL * N * (gram_k(n)) * 2 * sizeof(T));
     id = prof_.start();
     // The S1/S2 sums came with the Gram pass (one partial per Gram block);
-    // the cross S1 sums take their own pass.
+    // the cross S1 sums take their own pass.  One launch reduces them all.
+    std::vector<PartSum> sums{{gpart_[n].data(), nb, m * 2, gsum_[n].data()}};
+    if (moments) sums.push_back({gpart2_[n].data(), nb, m, gsum2_[n].data()});
     if (cross_) launch_zcross<T>(N, Bs_, z_of(n), nblk_z_[n], zpart_[n].data(), mv, s_);
-    launch_reduce_parts(zpart_[n].data(), cross_ ? nblk_z_[n] : nb, rows * kL * 4, zsum_[n].data(), s_);
+    sums.push_back({zpart_[n].data(), cross_ ? nblk_z_[n] : nb, rows * kL * 4, zsum_[n].data()});
     if (n == 0 && !cross_) {
       launch_meanvar<T>(N, B_, f_->maps[0].data(), nblk_mv_, mvpart_.data(), mv, s_);
-      launch_reduce_parts(mvpart_.data(), nblk_mv_, rows * 4, mvsum_.data(), s_);
+      sums.push_back({mvpart_.data(), nblk_mv_, rows * 4, mvsum_.data()});
     }
-    // The S1/S2 sums come with the Gram pass: this is the reduction of their
-    // partials, the cross S1 pass over z and level 0's mean / variance pass.
+    launch_reduce_parts(sums, s_);
+    // This timer holds the reductions, the cross S1 pass over z and level 0's
+    // mean / variance pass; the bytes are the latter two's and the S1/S2 partials'.
     double zbytes = double(cross_ ? nblk_z_[n] : nb) * rows * kL * 4 * 8.0 + double(rows) * kL * 4 * 8.0;
     if (cross_) zbytes += double(B_) * kL * N * 2 * sizeof(T);
     if (n == 0 && !cross_) zbytes += double(B_) * N * sizeof(T) + double(nblk_mv_ + 1) * rows * 4 * 8.0;
@@ -1107,11 +1095,11 @@ class EngineT final : public Engine {
   struct GraphEntry {
     const void* ptr;
     bool flag;
-    std::array<hipGraphExec_t, 8> exec{};  // one graph, or the steps of a split sweep
+    std::array<hipGraphExec_t, 12> exec{};  // one graph, or the steps of a split sweep
     int count = 0;
   };
   static constexpr size_t kMaxGraphs = 8;
-  static constexpr int kMaxSteps = 8;
+  static constexpr int kMaxSteps = 12;
 
   template <typename Body>
   hipGraph_t capture(Body&& body) {
@@ -1199,60 +1187,114 @@ class EngineT final : public Engine {
     STL_HIP(e1);
   }
 
-  // The forward's steps.  After level n's z convolution (and the moduli it
-  // completes), levels > n need nothing more from level n, and level n's
-  // branch convolution and sums need nothing from them: levels 0 and 1's
-  // sums run on side streams beside the coarser levels.
+  // Whether the sweeps run in few steps (below): up to the pixels of one map
+  // at nside 128.  Few against all steps, us for a forward with its gradient:
+  // nside 64 FP64 560 / 637, 128 FP64 948 / 977, 128 mixed 770 / 798, but 2
+  // maps at 128 mixed 1023 / 935, 256 mixed 1414 / 1321.
+  bool few_steps() const { return int64_t(B_) * N_[0] <= 12 * 128 * 128; }
+
+  // First level that takes no launches of its own.
+  int batch_from() const { return batch_on() ? qc_ : levels_; }
+
+  // The forward's steps.  Level n's z convolution needs the decimated maps
+  // only, and level n's branch convolution and sums need nothing from the
+  // coarser levels, which need nothing from them: what is in line on the
+  // engine stream is the z convolutions with the moduli's decimations, level
+  // by level; the maps' decimations (with the batched levels' z convolutions)
+  // run beside level 0's z convolution, the sums of the levels on the side
+  // streams.
   std::vector<Step> forward_steps(const double* x_dev, bool moments) {
-    // The maps' decimations are not needed by level 0: they follow the fork.
-    auto first = [this, x_dev] {
-      load_maps(x_dev);
-      fwd_z(0);
-    };
-    auto dec_all = [this] {
+    auto load = [this, x_dev] { load_maps(x_dev); };
+    auto decs = [this, moments] {
       for (int n = 1; n < levels_; ++n) dec_maps(n);
+      if (batch_on()) run_batches(qfwd_[moments ? 1 : 0], 0, 1);  // the batched levels' z convolutions
     };
-    auto coarser = [this, moments](int from) { return [this, moments, from] { fwd_levels(from, moments); }; };
-    auto sums = [this, moments](int n) { return [this, moments, n] { fwd_sums(n, moments); }; };
+    auto zs = [this](int from, int to) {
+      return [this, from, to] {
+        for (int n = from; n < to; ++n) fwd_z(n);
+      };
+    };
+    auto sums = [this, moments](int from, int to) {
+      return [this, moments, from, to] {
+        for (int n = from; n < to; ++n) fwd_sums(n, moments);
+      };
+    };
     auto finish = [this, moments] { fwd_finish(moments); };
     // The recompute store holds one level's z and branches: the levels in turn.
     if (f_->recompute)
       return {{[this, x_dev, moments] { enqueue_forward(x_dev, moments); }, 0, {}}};
-    if (levels_ == 1) return {{[first, sums, finish] { first(); sums(0)(); finish(); }, 0, {}}};
-    if (levels_ == 2)
-      return {{first, 0, {}},
-              {sums(0), 1, {0}},
-              {[dec_all, coarser] {
-                 dec_all();
-                 coarser(1)();
-               },
-               0, {}},
-              {finish, 0, {1}}};
-    return {{first, 0, {}},
-            {sums(0), 1, {0}},
-            {[this, dec_all] {
-               dec_all();
-               fwd_z(1);
-             },
-             0, {}},
-            {sums(1), 2, {2}},
-            {coarser(2), 0, {}},
-            {finish, 0, {1, 3}}};
+    if (levels_ == 1)
+      return {{[load, zs, sums, finish] { load(); zs(0, 1)(); sums(0, 1)(); finish(); }, 0, {}}};
+    const int mid = batch_from();
+    const std::vector<Batch>& batch = qfwd_[moments ? 1 : 0];
+    // Small maps: a graph launch costs the host about as much as its kernels
+    // take, so few of them, what is in line first.  A batch ends with its
+    // branch convolutions, sums and reductions.
+    if (few_steps()) {
+      const size_t line = batch_on() ? batch.size() - 3 : 0;  // z and the moduli's decimations
+      auto in_line = [this, load, decs, zs, mid, line, &batch] {
+        load();
+        decs();
+        zs(0, mid)();
+        if (batch_on()) run_batches(batch, 1, line);
+      };
+      std::vector<Step> st{{in_line, 0, {}}, {sums(0, mid), 1, {0}}};
+      if (batch_on()) st.push_back({[this, line, &batch] { run_batches(batch, line); }, 0, {}});
+      st.push_back({finish, 0, {1}});
+      return st;
+    }
+    std::vector<Step> st{{load, 0, {}}, {decs, 2, {0}}, {zs(0, 1), 0, {}}, {sums(0, 1), 1, {2}}, {zs(1, 2), 0, {1}},
+                         {sums(1, 2), 2, {4}}};
+    int last = 5;  // the step that ends the second side stream
+    if (mid > 2) {
+      st.push_back({zs(2, mid), 0, {}});
+      st.push_back({sums(2, mid), 2, {6}});
+      last = 7;
+    }
+    if (batch_on()) st.push_back({[this, &batch] { run_batches(batch, 1); }, 0, {}});
+    st.push_back({finish, 0, {3, last}});
+    return st;
   }
 
   // The reverse's steps.  Level n's gV and branch adjoint read only level-n
-  // fields and the prelude's operands, and write level-n buffers: levels 0
-  // and 1's run on side streams beside the coarser levels; their chains
-  // (which need the coarser chain) follow on the engine stream.
+  // fields and the prelude's operands, and write level-n buffers: they run on
+  // side streams (level 0's on one, the others', coarse to fine, on the other)
+  // beside the batched levels and the chains, which need the coarser chain
+  // and follow on the engine stream.
   std::vector<Step> reverse_steps(double* grad_dev) {
-    auto coarser = [this](int down_to) { return [this, down_to] { rev_levels(down_to); }; };
-    auto last = [this, grad_dev] { rev_chain(0, grad_dev); };
-    auto prelude = [this] { rev_prelude(); };
+    auto branches = [this](int from, int to) {  // coarse to fine
+      return [this, from, to] {
+        for (int n = to - 1; n >= from; --n) rev_branch(n);
+      };
+    };
+    auto chains = [this](int from, int to) {
+      return [this, from, to] {
+        for (int n = to - 1; n >= from; --n) rev_chain(n);
+      };
+    };
     if (levels_ == 1 || f_->recompute) return {{[this, grad_dev] { sweep_reverse(grad_dev); }, 0, {}}};
-    if (levels_ == 2)
-      return {{prelude, 0, {}}, {[this] { rev_branch(0); }, 1, {0}}, {coarser(1), 0, {}}, {last, 0, {1}}};
-    return {{prelude, 0, {}},        {[this] { rev_branch(0); }, 1, {0}}, {[this] { rev_branch(1); }, 2, {0}},
-            {coarser(2), 0, {}},     {[this] { rev_chain(1); }, 0, {2}},  {last, 0, {1}}};
+    const int mid = batch_from();
+    if (few_steps()) {
+      std::vector<Step> st{{[this] { rev_prelude(); }, 0, {}}};
+      if (batch_on()) st.push_back({[this] { run_batches(qrev_); }, 0, {}});
+      st.push_back({branches(0, mid), 1, {0}});
+      st.push_back({[this, chains, mid, grad_dev] {
+                      chains(1, mid)();
+                      rev_chain(0, grad_dev);
+                    },
+                    0, {int(st.size()) - 1}});
+      return st;
+    }
+    std::vector<Step> st{{[this] { rev_prelude(); }, 0, {}}, {branches(0, 1), 1, {0}}};
+    if (mid > 2) st.push_back({branches(2, mid), 2, {0}});
+    const int coarse = int(st.size()) - 1;
+    st.push_back({branches(1, 2), 2, {0}});
+    const int one = int(st.size()) - 1;
+    if (batch_on()) st.push_back({[this] { run_batches(qrev_); }, 0, {}});
+    if (mid > 2) st.push_back({chains(2, mid), 0, {coarse}});
+    st.push_back({chains(1, 2), 0, {one}});
+    st.push_back({[this, grad_dev] { rev_chain(0, grad_dev); }, 0, {1}});
+    return st;
   }
 
   // Convolution kernel variant per level and kernel (forward z, forward
@@ -1368,8 +1410,9 @@ class EngineT final : public Engine {
   }
 
   // The batched launches of a sweep, in order, on the engine stream.
-  void run_batches(const std::vector<Batch>& batches) {
-    for (const Batch& b : batches) {
+  void run_batches(const std::vector<Batch>& batches, size_t first = 0, size_t last = SIZE_MAX) {
+    for (size_t i = first; i < std::min(last, batches.size()); ++i) {
+      const Batch& b = batches[i];
       int id = prof_.start();
       launch_batch<T>(b.tasks.data(), b.ntasks, b.items, b.lds, q_workgroups_, s_);
       prof_.stop(id, b.name, b.bytes);
@@ -1494,36 +1537,36 @@ class EngineT final : public Engine {
       v.in0 = f_->br[n].data();
       v.in1 = f_->z[n].data();
       v.in2 = dH_[n].data();
-      v.out0 = f_->qgbr[n].data();
-      v.out1 = f_->qgzp[n].data();
+      v.out0 = f_->lgbr[n].data();
+      v.out1 = f_->lgzp[n].data();
       vs.tasks.push_back(v);
       vs.bytes += double(B_) * N * ((n + 1) * kL * kL + kL) * 2 * sizeof(T) * 2;
       LevelTask<T> a = base(kQConvAdj4, n, (n + 1) * B_, split_blocks(N));
       a.conv = conv;
-      a.in0 = f_->qgbr[n].data();
-      a.out0 = f_->qchain[n].data();
+      a.in0 = f_->lgbr[n].data();
+      a.out0 = f_->lchain[n].data();
       as.tasks.push_back(a);
       as.bytes += conv_bytes(n, kL, (n + 1) * B_, true);
       if (conv.nfix > 0) {
         LevelTask<T> f = base(kQFix4, n, (n + 1) * B_, blocks(int64_t(conv.nfix) * kL, 256));
         f.conv = conv;
-        f.in0 = f_->qgbr[n].data();
-        f.out0 = f_->qchain[n].data();
+        f.in0 = f_->lgbr[n].data();
+        f.out0 = f_->lchain[n].data();
         fs.tasks.push_back(f);
       }
       if (n + 1 < levels_) {
         const DecOp<T> dec = dec_[n]->store.view();
         LevelTask<T> c = base(kQDecAdj4, n, (n + 1) * B_, blocks(dec.Rf * 4, 256));
         c.dec = dec;
-        c.in0 = f_->qchain[n + 1].data();
-        c.in1 = f_->qchain[n].data();
-        c.out0 = f_->qchain[n].data();
+        c.in0 = f_->lchain[n + 1].data();
+        c.in1 = f_->lchain[n].data();
+        c.out0 = f_->lchain[n].data();
         chain.push_back(Step{{c}, dec_bytes(n, kL, (n + 1) * B_, true), tag("batch_dec_adj", n)});
       }
       LevelTask<T> z = base(kQGz, n, B_, blocks(N, 256));
       z.in0 = f_->z[n].data();
-      z.in1 = f_->qgzp[n].data();
-      z.in2 = f_->qchain[n].data();
+      z.in1 = f_->lgzp[n].data();
+      z.in2 = f_->lchain[n].data();
       z.s1 = ds1_[n].data();
       z.s2 = ds2_[n].data();
       z.out0 = f_->qgz[n].data();

@@ -2431,23 +2431,32 @@ __device__ __forceinline__ void reduce_parts_body(const double* __restrict__ par
   }
 }
 
-__global__ __launch_bounds__(64 * kRedWaves) void k_reduce_parts(const double* __restrict__ part, int nblk,
-                                                                 int64_t m, double* __restrict__ out) {
+// first[i]: the first workgroup of array i (first[n]: past the last).
+struct PartSums {
+  PartSum sum[4];
+  int64_t first[5];
+  int n;
+};
+
+__global__ __launch_bounds__(64 * kRedWaves) void k_reduce_parts(PartSums ps) {
   __shared__ double sh[kRedWaves][64];
+  int a = 0;
+  while (a + 1 < ps.n && int64_t(blockIdx.x) >= ps.first[a + 1]) ++a;
+  const PartSum& p = ps.sum[a];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t i = blockIdx.x * int64_t(64) + lane;
+  const int64_t i = (blockIdx.x - ps.first[a]) * 64 + lane;
   double s = 0.0;
-  if (i < m) {
+  if (i < p.m) {
 #pragma unroll 8
-    for (int b = w; b < nblk; b += kRedWaves) s += part[size_t(b) * m + i];
+    for (int b = w; b < p.nblk; b += kRedWaves) s += p.part[size_t(b) * p.m + i];
   }
   sh[w][lane] = s;
   __syncthreads();
-  if (w == 0 && i < m) {
+  if (w == 0 && i < p.m) {
     double t = 0.0;
 #pragma unroll
     for (int k = 0; k < kRedWaves; ++k) t += sh[k][lane];
-    out[i] = t;
+    p.out[i] = t;
   }
 }
 
@@ -3455,8 +3464,15 @@ void launch_mask_combine(int B, int K, int R, int C, int64_t E, const uint64_t* 
   STL_HIP(hipGetLastError());
 }
 
-void launch_reduce_parts(const double* part, int nblk, int64_t m, double* out, hipStream_t s) {
-  k_reduce_parts<<<nblocks(m, 64), 64 * kRedWaves, 0, s>>>(part, nblk, m, out);
+void launch_reduce_parts(const std::vector<PartSum>& sums, hipStream_t s) {
+  PartSums ps{};
+  STL_CHECK(!sums.empty() && sums.size() <= 4, "reduction: 1 to 4 arrays");
+  for (const PartSum& p : sums) {
+    ps.sum[ps.n] = p;
+    ps.first[ps.n + 1] = ps.first[ps.n] + int64_t(nblocks(p.m, 64));
+    ++ps.n;
+  }
+  k_reduce_parts<<<unsigned(ps.first[ps.n]), 64 * kRedWaves, 0, s>>>(ps);
   STL_HIP(hipGetLastError());
 }
 

@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace stl {
@@ -97,8 +99,15 @@ void launch_zstats(int64_t N, int B, const cplx_t<T>* z, int nblk, double* part,
 // mean/var sums of the level-0 map: part [nblk][B * K][4] = (sum x, sum x^2, sum x^2, sum x^4).
 template <typename T>
 void launch_meanvar(int64_t N, int B, const T* x, int nblk, double* part, const MaskView& mask, hipStream_t s);
-// Sums the partials over blocks in block order: part [nblk][m] -> out [m].
-void launch_reduce_parts(const double* part, int nblk, int64_t m, double* out, hipStream_t s);
+// Sums of partials over blocks in block order, part [nblk][m] -> out [m], for
+// at most 4 arrays in one launch.
+struct PartSum {
+  const double* part;
+  int nblk;
+  int64_t m;
+  double* out;
+};
+void launch_reduce_parts(const std::vector<PartSum>& sums, hipStream_t s);
 
 // Statistics from the sky-wide sums, on the device: value i of row r =
 // b K + k (map b, mask k) is (src[arr][re + r bs] + i src[arr][im + r bs]) / Nd

@@ -325,6 +325,25 @@ def test_graph_replays_match_eager_launches(J):
             assert torch.equal(out_g, out_e)
 
 
+@pytest.mark.parametrize("nside,J,batch,batch_nside", [(128, 4, 1, 0), (32, 2, 17, 0), (32, 4, 17, 0), (32, 4, 17, 16),
+                                                       (16, 3, 64, 16), (32, 4, 16, 32)])
+def test_sweep_schedules_match_eager_launches(nside, J, batch, batch_nside):
+    """The graph steps over the streams, few of them up to 12 * 128^2 pixels
+    and one per level's part above, with no, some and all coarse levels in
+    batched launches, give the bits of the same kernels launched in turn."""
+    from stl_port import NativeEngine
+    print(f"[gpu] schedule nside={nside} J={J} batch={batch} batch_nside={batch_nside}", flush=True)
+    rng = np.random.default_rng(22)
+    opts = dict(batch=batch, precision="fp64", batch_nside=batch_nside, conv_variant=0)
+    with NativeEngine(nside, J, **opts) as g, NativeEngine(nside, J, timing=True, **opts) as e:
+        cots = rng.standard_normal((batch, g.ncoeff)) + 1j * rng.standard_normal((batch, g.ncoeff))
+        for it in range(3):
+            x = rng.standard_normal((batch, 12 * nside * nside))
+            for a, b in zip(g.forward(x, generation=it, moments=it == 1), e.forward(x, generation=it, moments=it == 1)):
+                np.testing.assert_array_equal(a, b)
+            np.testing.assert_array_equal(g.vjp(cots, generation=it), e.vjp(cots, generation=it))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_forward_conv_variants_agree(precision):
     """The convolution kernel variants (16 x 16 tiles, several faces per
