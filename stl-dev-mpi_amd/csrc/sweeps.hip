@@ -2513,6 +2513,111 @@ __global__ void k_mask_combine(int B, int K, int R, int C, int64_t E, const uint
   out[t] = acc;
 }
 
+// Lane k of each group of 4 lanes, to all 4.
+__device__ __forceinline__ double quad_lane(double v, int k) {
+  switch (k) {
+    case 0: return dpp_f64<0x00>(v);
+    case 1: return dpp_f64<0x55>(v);
+    case 2: return dpp_f64<0xAA>(v);
+    default: return dpp_f64<0xFF>(v);
+  }
+}
+__device__ __forceinline__ double quad_sum(double v) {
+  v += dpp_f64<0xB1>(v);         // lanes 0 1 | 2 3
+  return v + dpp_f64<0x4E>(v);   // the two pairs
+}
+
+// gV = H V (ADJ: H^H V) of U pixels per group of 4 lanes, FP64: lane l1
+// holds and forms the entries (d, l1) of all NL branch directions, so that
+// the loads and stores of the group's 4 lanes are one pixel's 4 orientations
+// and a wavefront's are contiguous; the others' entries come over DPP.  The z
+// row is split over the 4 lanes and summed.  store(d, u, value): entry
+// (d, l1), d = NL the z part.
+template <int NL, int U, bool ADJ, typename Store>
+__device__ __forceinline__ void gv_quad(const double2* Hs, const double2 (&V)[NL][U], const double2 (&zv)[U], int l1,
+                                        const Store& store) {
+  constexpr int K = NL * kL + 1;
+  auto mac = [&](double2& o, int i, int j, const double2& v) {
+    const double2 h = Hs[ADJ ? j * K + i : i * K + j];
+    if (ADJ) {
+      o.x += h.x * v.x + h.y * v.y;
+      o.y += h.x * v.y - h.y * v.x;
+    } else {
+      o.x += h.x * v.x - h.y * v.y;
+      o.y += h.x * v.y + h.y * v.x;
+    }
+  };
+  double2 o[U];
+#pragma unroll 1
+  for (int d = 0; d < NL; ++d) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) o[u] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        mac(o[u], d * kL + l1, j,
+            j == K - 1 ? zv[u] : make_double2(quad_lane(V[j / kL][u].x, j % kL), quad_lane(V[j / kL][u].y, j % kL)));
+#pragma unroll
+    for (int u = 0; u < U; ++u) store(d, u, o[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    o[u] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int d = 0; d < NL; ++d) mac(o[u], K - 1, d * kL + l1, V[d][u]);
+    if (l1 == 0) mac(o[u], K - 1, K - 1, zv[u]);
+    store(NL, u, make_double2(quad_sum(o[u].x), quad_sum(o[u].y)));
+  }
+}
+
+// Pixels per lane group, which share the reads of H: as many as the entries'
+// registers allow.
+constexpr int gv_px(int NL) { return NL == 1 ? 4 : NL <= 3 ? 2 : 1; }
+
+// Reverse of the Gram products of row b (CROSS: of the map pair 2b, 2b + 1:
+// with H the cotangent of G = V_a V_b^H, gV_a = H V_b and gV_b = H^H V_a):
+// the branch cotangents and z parts; one mask class, H [B kL][K][K] staged in
+// LDS.  Bound by memory at the fine levels.  With a thread per pixel the
+// 64-byte strides between lanes held it at 4.9 TB/s, and the reads of H (a
+// 16-byte broadcast per 4 fma) held the pair's at 3.4: nside 256 level 0, one
+// map 103 -> 85 us (5.9 TB/s), level 1 54 -> 43; a pair 300 -> 179, level 1
+// 148 -> 87, level 6 51 -> 21.
+template <int NL, bool CROSS>
+__global__ __launch_bounds__(256) void k_gv_quad(int64_t N, int Bf, const double2* __restrict__ br,
+                                                 const double2* __restrict__ z, const double2* __restrict__ H,
+                                                 double2* __restrict__ gbr, double2* __restrict__ gzp) {
+  constexpr int K = NL * kL + 1, U = gv_px(NL), C = CROSS ? 2 : 1;
+  __shared__ double2 Hs[K * K];
+  const int bl = blockIdx.y;  // b kL + l3
+  const int b = bl / kL, l3 = bl % kL, l1 = threadIdx.x % kL;
+  int64_t p[U];
+  double2 V[C][NL][U], zv[C][U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    p[u] = (blockIdx.x * int64_t(U) + u) * (256 / kL) + threadIdx.x / kL;
+    const int64_t pc = min(p[u], N - 1);  // all 4 lanes of a group hold a pixel
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int row = C * b + c;
+#pragma unroll
+      for (int d = 0; d < NL; ++d) V[c][d][u] = br[(((size_t(d) * Bf + row) * kL + l3) * N + pc) * kL + l1];
+      zv[c][u] = z[(size_t(row) * kL + l3) * N + pc];
+    }
+  }
+  for (int e = threadIdx.x; e < K * K; e += blockDim.x) Hs[e] = H[size_t(bl) * K * K + e];
+  __syncthreads();
+  auto to_row = [&](int row) {
+    return [=, &p](int d, int u, double2 v) {
+      if (p[u] >= N) return;
+      if (d < NL) gbr[(((size_t(d) * Bf + row) * kL + l3) * N + p[u]) * kL + l1] = v;
+      else if (l1 == 0) gzp[(size_t(row) * kL + l3) * N + p[u]] = v;
+    };
+  };
+  gv_quad<NL, U, false>(Hs, V[C - 1], zv[C - 1], l1, to_row(C * b));
+  if (CROSS) gv_quad<NL, U, true>(Hs, V[0], zv[0], l1, to_row(C * b + 1));
+}
+
 // gV = H V of one pixel: writes the branch cotangents and the z part.
 template <typename T, int K>
 __device__ __forceinline__ void gv_apply(const double2* Hs, const double2 (&V)[K], int64_t N, int B, int b, int l3,
@@ -3401,9 +3506,33 @@ void launch_zcross(int64_t N, int B, const cplx_t<T>* z, int nblk, double* part,
   STL_HIP(hipGetLastError());
 }
 
+// FP64 with one mask class: lane groups (FP32's 8-byte entries and the
+// classes' own H do better with a thread per pixel: nside 1024 level 0 mixed
+// 803 us against 879, 2 maps at 256 with masks 208 against 240).
+template <bool CROSS>
+void launch_gv_quad(int n, int64_t N, int B, const double2* branch, const double2* z, const double2* H,
+                    double2* gbranch, double2* gz_part, hipStream_t s) {
+  const dim3 grid(nblocks(N, (256 / kL) * gv_px(n + 1)), B * kL);
+  const int Bf = CROSS ? 2 * B : B;
+  switch (n + 1) {
+#define STL_GV(NL) \
+  case NL: k_gv_quad<NL, CROSS><<<grid, 256, 0, s>>>(N, Bf, branch, z, H, gbranch, gz_part); break;
+    STL_GV(1) STL_GV(2) STL_GV(3) STL_GV(4) STL_GV(5) STL_GV(6) STL_GV(7) STL_GV(8) STL_GV(9) STL_GV(10)
+    STL_GV(11) STL_GV(12)
+#undef STL_GV
+    default: throw std::runtime_error("gv: too many levels");
+  }
+  STL_HIP(hipGetLastError());
+}
+
 template <typename T>
 void launch_gv_x(int n, int64_t N, int B, const cplx_t<T>* branch, const cplx_t<T>* z, const double2* H,
                  cplx_t<T>* gbranch, cplx_t<T>* gz_part, const MaskView& mask, hipStream_t s) {
+  if constexpr (std::is_same_v<T, double>)
+    if (mask.C == 1) {
+      launch_gv_quad<true>(n, N, B, branch, z, H, gbranch, gz_part, s);
+      return;
+    }
   dim3 grid(nblocks(N, 256), B * kL);
   const int K = (n + 1) * kL + 1;
   const size_t hbytes = size_t(mask.C) * K * K * sizeof(double2);
@@ -3494,6 +3623,11 @@ void launch_gv(int n, int64_t N, int B, const cplx_t<T>* branch, const cplx_t<T>
     STL_HIP(hipGetLastError());
     return;
   }
+  if constexpr (std::is_same_v<T, double>)
+    if (mask.C == 1) {
+      launch_gv_quad<false>(n, N, B, branch, z, H, gbranch, gz_part, s);
+      return;
+    }
   const size_t hbytes = size_t(mask.C) * K * K * sizeof(double2);
   const bool lds = hbytes <= 64 * 1024;
   switch (n + 1) {

@@ -344,6 +344,30 @@ def test_sweep_schedules_match_eager_launches(nside, J, batch, batch_nside):
             np.testing.assert_array_equal(g.vjp(cots, generation=it), e.vjp(cots, generation=it))
 
 
+@pytest.mark.parametrize("cross", [False, True])
+@pytest.mark.parametrize("nside,J", [(2, 1), (16, 4), (32, 5)])
+def test_gram_reverse_lane_groups_match_per_pixel(nside, J, cross):
+    """The Gram products' reverse in FP64: lane groups with one H for all
+    pixels (no masks) against a thread per pixel with its class's H (a mask of
+    the whole sky beside another), down to 12 pixels (less than a workgroup's).
+    Sums of at most 4 J + 1 <= 21 products in another order differ by less than
+    21 * 2^-52 of their terms, 1e-13 allows their cancellation a factor of 20."""
+    from stl_port import NativeEngine
+    print(f"[gpu] gram reverse nside={nside} J={J} cross={cross}", flush=True)
+    rng = np.random.default_rng(23)
+    npix = 12 * nside * nside
+    x = rng.standard_normal((2, 2, npix) if cross else (2, npix))
+    w = np.stack([np.ones(npix), (np.arange(npix) % 3 == 0).astype(float)])
+    opts = dict(batch=2, precision="fp64", cross=cross, batch_nside=0, conv_variant=0)
+    with NativeEngine(nside, J, **opts) as whole, NativeEngine(nside, J, masks=w, **opts) as masked:
+        v, _ = whole.forward(x)
+        cot = rng.standard_normal(v.shape) + 1j * rng.standard_normal(v.shape)
+        g = whole.vjp(cot)
+        masked.forward(x)
+        gm = masked.vjp(np.stack([cot, np.zeros_like(cot)], axis=1))
+    assert np.linalg.norm(g - gm) < 1e-13 * np.linalg.norm(gm)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_forward_conv_variants_agree(precision):
     """The convolution kernel variants (16 x 16 tiles, several faces per
