@@ -2618,6 +2618,69 @@ __global__ __launch_bounds__(256) void k_gv_quad(int64_t N, int Bf, const double
   if (CROSS) gv_quad<NL, U, true>(Hs, V[0], zv[0], l1, to_row(C * b + 1));
 }
 
+// Level 0 in FP32 (sums in FP64), one mask class: pairs of lanes, lane h the
+// orientations 2h and 2h + 1 of the pair's two pixels, 16 bytes a load and
+// store, H read once for both; lane h sums pixel h's z row, and every sum
+// keeps the order of the thread per pixel's.  Bound by memory: nside 1024
+// 803 us with a thread per pixel, 678 here (5.9 TB/s), 697 with 4 pixels.
+template <int PICK>
+__device__ __forceinline__ float pair_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), PICK, 0xF, 0xF, false));
+}
+__global__ __launch_bounds__(256) void k_gv_pair(int64_t N, const float2* __restrict__ br, const float2* __restrict__ z,
+                                                 const double2* __restrict__ H, float2* __restrict__ gbr,
+                                                 float2* __restrict__ gzp) {
+  constexpr int K = kL + 1, U = 2;
+  __shared__ double2 Hs[K * K];
+  const size_t bl = blockIdx.y;  // b kL + l3
+  const int h = threadIdx.x & 1;
+  int64_t p[U];
+  float4 V[U];
+  float2 zv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    p[u] = (blockIdx.x * int64_t(U) + u) * 128 + threadIdx.x / 2;
+    const int64_t pc = min(p[u], N - 1);  // both lanes of a pair hold a pixel
+    V[u] = reinterpret_cast<const float4*>(br)[(bl * N + pc) * 2 + h];
+    zv[u] = z[bl * N + pc];
+  }
+  if (threadIdx.x < K * K) Hs[threadIdx.x] = H[bl * K * K + threadIdx.x];
+  __syncthreads();
+  // Entry j of pixel u, to both lanes.
+  auto entry = [&](int j, int u) {
+    if (j == K - 1) return zv[u];
+    const float x = j & 1 ? V[u].z : V[u].x, y = j & 1 ? V[u].w : V[u].y;
+    return j & 2 ? make_float2(pair_lane<0xF5>(x), pair_lane<0xF5>(y))
+                 : make_float2(pair_lane<0xA0>(x), pair_lane<0xA0>(y));
+  };
+  auto mac = [&](double2& o, const double2& hv, const float2& f) {
+    const double2 v = make_double2(double(f.x), double(f.y));
+    o.x += hv.x * v.x - hv.y * v.y;
+    o.y += hv.x * v.y + hv.y * v.x;
+  };
+  double2 o[2][U], oz = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) o[0][u] = o[1][u] = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const float2 f0 = entry(j, 0), f1 = entry(j, 1);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const double2 hv = Hs[(2 * h + r) * K + j];
+      mac(o[r][0], hv, f0);
+      mac(o[r][1], hv, f1);
+    }
+    mac(oz, Hs[(K - 1) * K + j], make_float2(h ? f1.x : f0.x, h ? f1.y : f0.y));
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (p[u] < N)
+      reinterpret_cast<float4*>(gbr)[(bl * N + p[u]) * 2 + h] =
+          make_float4(float(o[0][u].x), float(o[0][u].y), float(o[1][u].x), float(o[1][u].y));
+  const int64_t pz = h ? p[1] : p[0];
+  if (pz < N) gzp[bl * N + pz] = make_float2(float(oz.x), float(oz.y));
+}
+
 // gV = H V of one pixel: writes the branch cotangents and the z part.
 template <typename T, int K>
 __device__ __forceinline__ void gv_apply(const double2* Hs, const double2 (&V)[K], int64_t N, int B, int b, int l3,
@@ -3506,9 +3569,10 @@ void launch_zcross(int64_t N, int B, const cplx_t<T>* z, int nblk, double* part,
   STL_HIP(hipGetLastError());
 }
 
-// FP64 with one mask class: lane groups (FP32's 8-byte entries and the
-// classes' own H do better with a thread per pixel: nside 1024 level 0 mixed
-// 803 us against 879, 2 maps at 256 with masks 208 against 240).
+// FP64 with one mask class: lane groups (FP32's 8-byte entries are worse in
+// groups of 4 and the classes' own H does better with a thread per pixel:
+// nside 1024 level 0 mixed 879 us against 803, 2 maps at 256 with masks 240
+// against 208).
 template <bool CROSS>
 void launch_gv_quad(int n, int64_t N, int B, const double2* branch, const double2* z, const double2* H,
                     double2* gbranch, double2* gz_part, hipStream_t s) {
@@ -3626,6 +3690,14 @@ void launch_gv(int n, int64_t N, int B, const cplx_t<T>* branch, const cplx_t<T>
   if constexpr (std::is_same_v<T, double>)
     if (mask.C == 1) {
       launch_gv_quad<false>(n, N, B, branch, z, H, gbranch, gz_part, s);
+      return;
+    }
+  if constexpr (std::is_same_v<T, float>)
+    // Level 0 (coarser levels are bound by the reads of H, 420 us against
+    // 395 at nside 1024 level 1).
+    if (mask.C == 1 && n == 0) {
+      k_gv_pair<<<dim3(nblocks(N, 256), B * kL), 256, 0, s>>>(N, branch, z, H, gbranch, gz_part);
+      STL_HIP(hipGetLastError());
       return;
     }
   const size_t hbytes = size_t(mask.C) * K * K * sizeof(double2);

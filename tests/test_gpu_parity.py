@@ -368,6 +368,28 @@ def test_gram_reverse_lane_groups_match_per_pixel(nside, J, cross):
     assert np.linalg.norm(g - gm) < 1e-13 * np.linalg.norm(gm)
 
 
+@pytest.mark.parametrize("nside", [1, 2, 16])
+def test_gram_reverse_lane_pairs_match_per_pixel(nside):
+    """The same for level 0 in FP32, pairs of lanes: the sums of 5 products are
+    FP64 in the same order, rounded to FP32 once; the two engines' H differ by
+    rounding (2^-52), so single FP32 roundings (2^-24 of one value) may flip:
+    norms within 2^-24."""
+    from stl_port import NativeEngine
+    print(f"[gpu] gram reverse pairs nside={nside}", flush=True)
+    rng = np.random.default_rng(24)
+    npix = 12 * nside * nside
+    x = rng.standard_normal((3, npix))
+    w = np.stack([np.ones(npix), (np.arange(npix) % 3 == 0).astype(float)])
+    opts = dict(batch=3, precision="mixed", batch_nside=0, conv_variant=0)
+    with NativeEngine(nside, 1, **opts) as whole, NativeEngine(nside, 1, masks=w, **opts) as masked:
+        v, _ = whole.forward(x)
+        cot = rng.standard_normal(v.shape) + 1j * rng.standard_normal(v.shape)
+        g = whole.vjp(cot)
+        masked.forward(x)
+        gm = masked.vjp(np.stack([cot, np.zeros_like(cot)], axis=1))
+    assert np.linalg.norm(g - gm) < 2.0 ** -24 * np.linalg.norm(gm)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_forward_conv_variants_agree(precision):
     """The convolution kernel variants (16 x 16 tiles, several faces per
