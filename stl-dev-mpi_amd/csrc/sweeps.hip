@@ -2527,6 +2527,97 @@ __device__ __forceinline__ double quad_sum(double v) {
   return v + dpp_f64<0x4E>(v);   // the two pairs
 }
 
+// The pair's Gram products at levels 0 and 1 (K = 5, 9) in registers: lane l1
+// of a group of 4 holds a pixel's entries (d, l1) of both channels and sums
+// the rows (d, l1) of G, the other entries of channel b coming over DPP, and
+// its share of the z row.  Staged through LDS (k_gram_x, the coarser levels')
+// every product read its operands there: nside 256 FP64 level 0 155 -> 113
+// us, level 1 106 -> 60; level 2 (K = 13) takes too many registers, 83 us
+// against 36.  Several blocks' sums per row leave it at 2.2 TB/s.
+template <typename T, int NL, bool MOM, bool MASKED>
+__global__ __launch_bounds__(256) void k_gram_x_quad(int64_t N, int Bf, const cplx_t<T>* __restrict__ br,
+                                                     const cplx_t<T>* __restrict__ z, double* __restrict__ part,
+                                                     double* __restrict__ part2, MaskView mask) {
+  constexpr int K = NL * kL + 1, E = K * K, R = NL + 1;  // a lane's rows: (d, l1), then its share of z's
+  constexpr int M = MOM ? 3 : 2;
+  __shared__ double red[4][E][M];
+  const int bl = blockIdx.y;  // (b K + k) kL + l3
+  const int l3 = bl % kL, mk = (bl / kL) % mask.K, b = bl / (kL * mask.K);
+  const int l1 = threadIdx.x % kL;
+  double acc[NL][K][M] = {}, accz[R][M] = {};  // accz: z row at (d, l1), then at z
+  auto add = [](double (&o)[M], const double2& a, const double2& c) {
+    const double re = a.x * c.x + a.y * c.y, im = a.y * c.x - a.x * c.y;
+    o[0] += re;
+    o[1] += im;
+    if (MOM) o[M - 1] += re * re + im * im;
+  };
+  constexpr int U = NL == 1 ? 4 : 2;  // pixels whose loads travel together
+  for (int64_t p0 = blockIdx.x * int64_t(256 / kL); p0 < N; p0 += U * gridDim.x * int64_t(256 / kL)) {
+    cplx_t<T> V[U][2][R];
+    int64_t p[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      p[u] = p0 + u * gridDim.x * int64_t(256 / kL) + threadIdx.x / kL;
+      const int64_t pc = min(p[u], N - 1);  // all 4 lanes of a group hold a pixel
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int d = 0; d < NL; ++d) V[u][c][d] = br[(((size_t(d) * Bf + 2 * b + c) * kL + l3) * N + pc) * kL + l1];
+        V[u][c][NL] = z[(size_t(2 * b + c) * kL + l3) * N + pc];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // Channel a outside the mask (and past the end): its products add nothing.
+      const bool in = p[u] < N && (!MASKED || in_mask(mask, p[u], mk));
+      double2 a[R], c[R];
+#pragma unroll
+      for (int d = 0; d < R; ++d) {
+        a[d] = in ? to_d2<T>(V[u][0][d]) : make_double2(0.0, 0.0);
+        c[d] = to_d2<T>(V[u][1][d]);
+      }
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        const double2 cj =
+            j == K - 1 ? c[NL] : make_double2(quad_lane(c[j / kL].x, j % kL), quad_lane(c[j / kL].y, j % kL));
+#pragma unroll
+        for (int d = 0; d < NL; ++d) add(acc[d][j], a[d], cj);
+      }
+#pragma unroll
+      for (int d = 0; d < R; ++d) add(accz[d], a[NL], c[d]);
+    }
+  }
+  // The wave's lanes of one l1, then the 4 waves in order.
+  const int wave = threadIdx.x / 64;
+  auto put = [&](int i, int j, const double (&o)[M], bool mine) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      double v = o[m];
+#pragma unroll
+      for (int x = 4; x < 64; x *= 2) v += __shfl_xor(v, x);
+      if (mine) red[wave][i * K + j][m] = v;
+    }
+  };
+  const bool first = threadIdx.x % 64 < kL;
+#pragma unroll
+  for (int d = 0; d < NL; ++d) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) put(d * kL + l1, j, acc[d][j], first);
+    put(K - 1, d * kL + l1, accz[d], first);
+  }
+  put(K - 1, K - 1, accz[NL], first && l1 == 0);
+  __syncthreads();
+  const size_t base = (size_t(blockIdx.x) * gridDim.y + bl) * E;
+  for (int e = threadIdx.x; e < E; e += 256) {
+    double v[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) v[m] = ((red[0][e][m] + red[1][e][m]) + red[2][e][m]) + red[3][e][m];
+    part[(base + e) * 2] = v[0];
+    part[(base + e) * 2 + 1] = v[1];
+    if (MOM) part2[base + e] = v[M - 1];
+  }
+}
+
 // gV = H V (ADJ: H^H V) of U pixels per group of 4 lanes, FP64: lane l1
 // holds and forms the entries (d, l1) of all NL branch directions, so that
 // the loads and stores of the group's 4 lanes are one pixel's 4 orientations
@@ -3089,9 +3180,6 @@ __device__ __forceinline__ void level_item(const LevelTask<T>& t, int64_t bx, in
   }
 }
 
-// Persistent workgroups take items in queue order; an item runs once the tasks
-// its task depends on have completed.  Every workgroup leaves once the items
-// are exhausted (the item counter only grows), so the grid always drains.
 // Workgroup w runs items w, w + grid, ...: the items of independent tasks,
 // each found by binary search over the tasks' first items.
 template <typename T>
@@ -3540,6 +3628,19 @@ template <typename T>
 void launch_gram_x(int n, int64_t N, int B, const cplx_t<T>* branch, const cplx_t<T>* z, bool moments, int nblk,
                    double* part, double* part2, const MaskView& mask, hipStream_t s) {
   const int K = (n + 1) * kL + 1;
+  if (n < 2) {
+    const dim3 qgrid(nblk, B * mask.K * kL);
+    auto go = [&](auto kernel) { kernel<<<qgrid, 256, 0, s>>>(N, 2 * B, branch, z, part, part2, mask); };
+#define STL_GRAMXQ(NL)                                                                                       \
+  case NL:                                                                                                   \
+    if (moments) go(mask.cls ? k_gram_x_quad<T, NL, true, true> : k_gram_x_quad<T, NL, true, false>);        \
+    else go(mask.cls ? k_gram_x_quad<T, NL, false, true> : k_gram_x_quad<T, NL, false, false>);              \
+    break;
+    switch (n + 1) { STL_GRAMXQ(1) STL_GRAMXQ(2) }
+#undef STL_GRAMXQ
+    STL_HIP(hipGetLastError());
+    return;
+  }
   const int BS = K <= 13 ? 2 : 4;
   const int KP = (K + BS - 1) / BS * BS, NR = KP / BS;
   STL_CHECK(NR * NR <= 256, "cross gram: too many levels");
