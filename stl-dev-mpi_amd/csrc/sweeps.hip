@@ -1519,40 +1519,82 @@ constexpr int kDecPre = 8;
 
 template <typename T>
 __device__ inline void dec_prefetch(const int16_t* __restrict__ off, const T* __restrict__ val, int64_t R, int cap,
-                                    int64_t r, int cnt, int s0, int16_t (&eo)[kDecPre], T (&ev)[kDecPre]) {
+                                    int64_t r, int cnt, int16_t (&eo)[kDecPre], T (&ev)[kDecPre]) {
 #pragma unroll
-  for (int u = 0; u < kDecPre; ++u) {
-    const size_t at = size_t(min(s0 + u, cap - 1)) * R + r;
-    eo[u] = off[at];
-    ev[u] = s0 + u < cnt ? val[at] : T(0);
+  for (int s = 0; s < kDecPre; ++s) {
+    const size_t at = size_t(min(s, cap - 1)) * R + r;
+    eo[s] = off[at];
+    ev[s] = s < cnt ? val[at] : T(0);
   }
 }
 
-// Sum of a row's entries over its staged window (planes of PLANE elements,
-// rows of SW): the first kDecPre entries are in eo / ev; each further chunk
-// loads while the previous one's products run (an entry at a time, its load
-// was waited for before the next one's was issued).
+// Products of a row's first entries (eo / ev) with its staged window (planes
+// of PLANE elements, rows of SW).
+template <typename T, int NI, int SW, int PLANE>
+__device__ __forceinline__ void dec_first(const int16_t (&eo)[kDecPre], const T (&ev)[kDecPre], const T* xs, int pos,
+                                          T (&acc)[NI]) {
+#pragma unroll
+  for (int u = 0; u < kDecPre; ++u) {
+    const int src = pos + off_dy(eo[u]) * SW + off_dx(eo[u]);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[j] = fma(ev[u], xs[j * PLANE + src], acc[j]);
+  }
+}
+
+// Sum of a coarse pixel's row, 24 to 32 entries: the first kDecPre are in eo /
+// ev; each further chunk loads while the previous one's products run (an entry
+// at a time, its load was waited for before the next one's was issued).  A row
+// loads no chunk past its entries (a chunk ahead for every row: nside 1024
+// FP64, level 1 380 us, 353 so); past the count a slot adds 0 * 0.
 template <typename T, int NI, int SW, int PLANE>
 __device__ __forceinline__ void dec_gather(const int16_t* __restrict__ off, const T* __restrict__ val, int64_t R,
                                            int cap, int64_t r, int cnt, int16_t (&eo)[kDecPre], T (&ev)[kDecPre],
                                            const T* xs, int pos, T (&acc)[NI]) {
-  for (int s0 = 0;; s0 += kDecPre) {
-    int16_t no[kDecPre];
-    T nv[kDecPre];
-    // Unconditional (slots clamped to the capacity), as in pipelined_slots.
-    dec_prefetch<T>(off, val, R, cap, r, cnt, s0 + kDecPre, no, nv);
+  int16_t no[kDecPre];
+  T nv[kDecPre];
+  auto load = [&](int s0) {
 #pragma unroll
     for (int u = 0; u < kDecPre; ++u) {
-      const int src = pos + off_dy(eo[u]) * SW + off_dx(eo[u]);
-#pragma unroll
-      for (int j = 0; j < NI; ++j) acc[j] = fma(ev[u], xs[j * PLANE + src], acc[j]);
+      const size_t at = size_t(min(s0 + u, cap - 1)) * R + r;
+      no[u] = off[at];
+      nv[u] = val[at];
     }
-    if (s0 + kDecPre >= cnt) return;
+  };
+  if (kDecPre < cnt) load(kDecPre);
+  dec_first<T, NI, SW, PLANE>(eo, ev, xs, pos, acc);
+  for (int s0 = kDecPre; s0 < cnt; s0 += kDecPre) {
 #pragma unroll
     for (int u = 0; u < kDecPre; ++u) {
       eo[u] = no[u];
       ev[u] = nv[u];
     }
+    if (s0 + kDecPre < cnt) load(s0 + kDecPre);
+#pragma unroll
+    for (int u = 0; u < kDecPre; ++u) {
+      const bool in = s0 + u < cnt;
+      const int src = pos + off_dy(eo[u]) * SW + off_dx(eo[u]);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[j] = fma(in ? ev[u] : T(0), in ? xs[j * PLANE + src] : T(0), acc[j]);
+    }
+  }
+}
+
+// The same an entry at a time: fine cells' rows, 5 to 9 entries, where nearly
+// all end with the first kDecPre (nside 1024 mixed, level 1: 93 us; in chunks
+// 112 with one ahead for every row, 105 for the rows that have one), and the
+// coarse rows of large launches (launch_dec_fwd).
+template <typename T, int NI, int SW, int PLANE>
+__device__ __forceinline__ void dec_gather_serial(const int16_t* __restrict__ off, const T* __restrict__ val, int64_t R,
+                                                  int64_t r, int cnt, int16_t (&eo)[kDecPre], T (&ev)[kDecPre],
+                                                  const T* xs, int pos, T (&acc)[NI]) {
+  dec_first<T, NI, SW, PLANE>(eo, ev, xs, pos, acc);
+  for (int s = kDecPre; s < cnt; ++s) {
+    const size_t at = size_t(s) * R + r;
+    const int16_t e = off[at];
+    const T v = val[at];
+    const int src = pos + off_dy(e) * SW + off_dx(e);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[j] = fma(v, xs[j * PLANE + src], acc[j]);
   }
 }
 
@@ -1578,7 +1620,7 @@ __device__ inline bool span_inside(int x0, int y0, int w, int order) {
 // face and one row; the fine window of their candidates, fine offsets
 // kDecLo..kDecHi around the tile's children ((2 TC + 8)^2 pixels), is staged
 // in LDS (planar [j][pixel]) and every entry reads it at its stored offset.
-template <typename T, int NI, int TC>
+template <typename T, int NI, int TC, bool CHUNKS>
 __global__ __launch_bounds__(TC * TC) void k_dec_fwd_tiled(DecOp<T> op, const T* __restrict__ x, int rows,
                                                            T* __restrict__ y) {
   constexpr int SW = 2 * TC + (kDecHi - kDecLo + 1) - 2, SA = SW * SW;
@@ -1594,7 +1636,7 @@ __global__ __launch_bounds__(TC * TC) void k_dec_fwd_tiled(DecOp<T> op, const T*
   const int cnt = op.cnt[r];
   int16_t eo[kDecPre];
   T ev[kDecPre];
-  dec_prefetch<T>(op.off, op.val, op.Rc, op.S, r, cnt, 0, eo, ev);
+  dec_prefetch<T>(op.off, op.val, op.Rc, op.S, r, cnt, eo, ev);
   const bool inside = span_inside(fx0, fy0, SW, op.order_f);
   stage_window<T, NI, SA, SA, TC * TC>(xr, xs, [&](int idx, int& lp) {
     int wx, wy;
@@ -1609,7 +1651,8 @@ __global__ __launch_bounds__(TC * TC) void k_dec_fwd_tiled(DecOp<T> op, const T*
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-  dec_gather<T, NI, SW, SA>(op.off, op.val, op.Rc, op.S, r, cnt, eo, ev, xs, pos, acc);
+  if constexpr (CHUNKS) dec_gather<T, NI, SW, SA>(op.off, op.val, op.Rc, op.S, r, cnt, eo, ev, xs, pos, acc);
+  else dec_gather_serial<T, NI, SW, SA>(op.off, op.val, op.Rc, r, cnt, eo, ev, xs, pos, acc);
   const int64_t p = int64_t(ti.face) * op.npf_c + ti.base + li;
 #pragma unroll
   for (int j = 0; j < NI; ++j) y[(size_t(row) * Nc + p) * NI + j] = acc[j];
@@ -1634,7 +1677,7 @@ __device__ __forceinline__ void dec_adj_tile(const DecOp<T>& op, const T* __rest
   const int cnt = op.tcnt[q];
   int16_t eo[kDecPre];
   T ev[kDecPre];
-  dec_prefetch<T>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, 0, eo, ev);
+  dec_prefetch<T>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, eo, ev);
   T base[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) base[j] = add ? add[o + j] : T(0);
@@ -1651,7 +1694,7 @@ __device__ __forceinline__ void dec_adj_tile(const DecOp<T>& op, const T* __rest
   T acc[NI];
 #pragma unroll
   for (int j = 0; j < NI; ++j) acc[j] = T(0);
-  dec_gather<T, NI, SW, SA>(op.toff, op.tval, op.Rf, op.Tn, q, cnt, eo, ev, gs, pos, acc);
+  dec_gather_serial<T, NI, SW, SA>(op.toff, op.tval, op.Rf, q, cnt, eo, ev, gs, pos, acc);
 #pragma unroll
   for (int j = 0; j < NI; ++j) h[j] = add ? acc[j] + base[j] : acc[j];
 }
@@ -3496,12 +3539,22 @@ void launch_dec_fwd(const DecOp<T>& op, int NI, const T* x, int rows, T* y, hipS
     STL_CHECK(op.S >= 1, "decimation: empty operator store");
     if (op.order_c >= 4) {
       dim3 grid(unsigned(op.Rc / 256 * 4 * rows));
-      if (NI == 1) k_dec_fwd_tiled<T, 1, 16><<<grid, 256, 0, s>>>(op, x, rows, y);
-      else k_dec_fwd_tiled<T, kL, 16><<<grid, 256, 0, s>>>(op, x, rows, y);
+      // One entry at a time where enough workgroups share a CU to hide the
+      // loads: the chunks' longer code then costs more than they save.
+      // serial / chunks, us: FP32 maps at 2304 workgroups 26.7 / 25.5, at
+      // 6144 46.0 / 47.2, at 49152 265 / 280, moduli at 49152 409 / 422; FP64
+      // maps at 1536 23.0 / 22.7, at 2112 29.1 / 30.6, at 49152 406 / 451.
+      // FP64 moduli, 3 workgroups a CU (LDS), gain at every size: 96 13.5 /
+      // 12.3, 49152 889 / 828.
+      auto go = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(op, x, rows, y); };
+      const bool serial = grid.x > 16384 / sizeof(T);
+      if (NI == 1) go(serial ? k_dec_fwd_tiled<T, 1, 16, false> : k_dec_fwd_tiled<T, 1, 16, true>);
+      else if constexpr (sizeof(T) == 8) go(k_dec_fwd_tiled<T, kL, 16, true>);
+      else go(serial ? k_dec_fwd_tiled<T, kL, 16, false> : k_dec_fwd_tiled<T, kL, 16, true>);
     } else {
       dim3 grid(unsigned(op.Rc / 64 * 4 * rows));
-      if (NI == 1) k_dec_fwd_tiled<T, 1, 8><<<grid, 64, 0, s>>>(op, x, rows, y);
-      else k_dec_fwd_tiled<T, kL, 8><<<grid, 64, 0, s>>>(op, x, rows, y);
+      if (NI == 1) k_dec_fwd_tiled<T, 1, 8, true><<<grid, 64, 0, s>>>(op, x, rows, y);
+      else k_dec_fwd_tiled<T, kL, 8, true><<<grid, 64, 0, s>>>(op, x, rows, y);
     }
     STL_HIP(hipGetLastError());
     return;

@@ -94,6 +94,51 @@ def test_operators_match_oracle(nside):
             assert rel(gd.cpu().numpy(), (D.T @ g.T).T) < 1e-13
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nside", [16, 32, 64, 128])
+def test_decimation_of_an_infinite_pixel(nside, precision):
+    """A row sums its own entries only: an infinite pixel gives an infinity (and no NaN) in every row
+    that holds it, and leaves the others at 0.  Rows of fewer than 8 entries are left out: the 8 slots
+    loaded ahead of the window may add 0 times the pixel at its centre there."""
+    from stl_port import NativeEngine
+    indptr, cols, vals = O.decimation_rows(nside, 0, 3 * nside * nside)
+    D = sp.csr_matrix((vals, cols, indptr), shape=(3 * nside * nside, 12 * nside * nside))
+    rng = np.random.default_rng(nside)
+    with NativeEngine(nside, 2, precision=precision) as eng:
+        for kind, A in ((2, D), (3, D.T.tocsr())):
+            big = abs(A) > 1e-12  # smaller weights may be rounded zeros
+            full = np.asarray(big.sum(axis=1)).ravel() >= 8
+            pixels = rng.choice(A.shape[1] // 4, 24, replace=False) * 4 + rng.integers(0, 4, 24)
+            pixels[:12] &= ~3  # first children, the centres of the coarse pixels' windows
+            x = np.zeros((24, A.shape[1]))
+            x[np.arange(24), pixels] = np.inf
+            print(f"[gpu] infinite pixel nside={nside} kind={kind} {precision}", flush=True)
+            y = torch.empty((24, A.shape[0]), dtype=torch.float64, device="cuda")
+            eng.apply_operator(kind, 0, torch.from_numpy(x).cuda(), y)
+            y, w = y.cpu().numpy(), A.tocsc()[:, pixels].toarray().T
+            held = big.tocsc()[:, pixels].toarray().T & full
+            assert held.sum() > 24
+            np.testing.assert_array_equal(y[held], np.sign(w[held]) * np.inf)
+            assert not y[(w == 0) & full].any()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_decimation_by_chunks_and_by_entries_agree(precision):
+    """24 maps take the decimation an entry at a time (4608 workgroups), 4 of them in chunks of
+    entries: the same products in the same order, the same bits."""
+    from stl_port import NativeEngine
+    nside = 128
+    x = torch.from_numpy(np.random.default_rng(1).standard_normal((24, 12 * nside * nside))).cuda()
+    with NativeEngine(nside, 2, precision=precision) as eng:
+        print(f"[gpu] decimation forms {precision}", flush=True)
+        y = torch.empty((24, 3 * nside * nside), dtype=torch.float64, device="cuda")
+        eng.apply_operator(2, 0, x, y)
+        for at in range(0, 24, 4):
+            part = torch.empty((4, 3 * nside * nside), dtype=torch.float64, device="cuda")
+            eng.apply_operator(2, 0, x[at:at + 4].contiguous(), part)
+            assert torch.equal(y[at:at + 4], part)
+
+
 @pytest.mark.parametrize("case", [c for c in cases("stats", "stats")
                                   if c["L"] == 4 and c["kernel_sz"] == 5 and c["channels"] == 1
                                   and not c["fewer"] and c["j_to_dg"] == list(range(c["J"]))],
