@@ -1187,22 +1187,25 @@ class EngineT final : public Engine {
     STL_HIP(e1);
   }
 
-  // Whether the sweeps run in few steps (below): up to the pixels of one map
-  // at nside 128.  Few against all steps, us for a forward with its gradient:
-  // nside 64 FP64 560 / 637, 128 FP64 948 / 977, 128 mixed 770 / 798, but 2
-  // maps at 128 mixed 1023 / 935, 256 mixed 1414 / 1321.
+  // With batched levels, whether the sweeps run in few steps (below): up to
+  // the pixels of one map at nside 128.  Few against all steps, us for a
+  // forward with its gradient: nside 64 FP64 545 / 608, 128 FP64 923 / 941,
+  // 128 mixed 746 / 772, but 5 maps at 64 FP64 990 / 912, 2 maps at 128 mixed
+  // 1011 / 923, 256 mixed 1389 / 1294.
   bool few_steps() const { return int64_t(B_) * N_[0] <= 12 * 128 * 128; }
-
-  // First level that takes no launches of its own.
-  int batch_from() const { return batch_on() ? qc_ : levels_; }
 
   // The forward's steps.  Level n's z convolution needs the decimated maps
   // only, and level n's branch convolution and sums need nothing from the
-  // coarser levels, which need nothing from them: what is in line on the
-  // engine stream is the z convolutions with the moduli's decimations, level
-  // by level; the maps' decimations (with the batched levels' z convolutions)
-  // run beside level 0's z convolution, the sums of the levels on the side
-  // streams.
+  // coarser levels, which need nothing from them.  With batched levels, what
+  // is in line on the engine stream is the z convolutions with the moduli's
+  // decimations, level by level; the maps' decimations (with the batched
+  // levels' z convolutions) run beside level 0's z convolution, the sums of
+  // the levels on the side streams.  Without (masks, cross statistics, few
+  // levels), levels 0 and 1's sums run on the side streams beside the coarser
+  // levels, level by level: every level's part on its own is slower there
+  // (us, this / all steps / few: 32 maps of 2 levels mixed 515 / 641 / 623 at
+  // nside 32; masks at 64 mixed 728 / 794 / 827; 2 maps at 256 with masks
+  // FP64 2940 / 3010 / 3282; 512 with masks mixed 3762 / 3919 / 4446).
   std::vector<Step> forward_steps(const double* x_dev, bool moments) {
     auto load = [this, x_dev] { load_maps(x_dev); };
     auto decs = [this, moments] {
@@ -1225,42 +1228,62 @@ class EngineT final : public Engine {
       return {{[this, x_dev, moments] { enqueue_forward(x_dev, moments); }, 0, {}}};
     if (levels_ == 1)
       return {{[load, zs, sums, finish] { load(); zs(0, 1)(); sums(0, 1)(); finish(); }, 0, {}}};
-    const int mid = batch_from();
+    if (!batch_on()) {
+      auto first = [load, zs] {
+        load();
+        zs(0, 1)();
+      };
+      auto second = [this, decs, zs, sums] {
+        decs();
+        zs(1, 2)();
+        if (levels_ == 2) sums(1, 2)();
+      };
+      std::vector<Step> st{{first, 0, {}}, {sums(0, 1), 1, {0}}, {second, 0, {}}};
+      if (levels_ > 2) {
+        st.push_back({sums(1, 2), 2, {2}});
+        st.push_back({[this, moments] { fwd_levels(2, moments); }, 0, {}});
+        st.push_back({finish, 0, {1, 3}});
+      } else {
+        st.push_back({finish, 0, {1}});
+      }
+      return st;
+    }
     const std::vector<Batch>& batch = qfwd_[moments ? 1 : 0];
     // Small maps: a graph launch costs the host about as much as its kernels
     // take, so few of them, what is in line first.  A batch ends with its
     // branch convolutions, sums and reductions.
     if (few_steps()) {
-      const size_t line = batch_on() ? batch.size() - 3 : 0;  // z and the moduli's decimations
-      auto in_line = [this, load, decs, zs, mid, line, &batch] {
+      const size_t line = batch.size() - 3;  // z and the moduli's decimations
+      auto in_line = [this, load, decs, zs, line, &batch] {
         load();
         decs();
-        zs(0, mid)();
-        if (batch_on()) run_batches(batch, 1, line);
+        zs(0, qc_)();
+        run_batches(batch, 1, line);
       };
-      std::vector<Step> st{{in_line, 0, {}}, {sums(0, mid), 1, {0}}};
-      if (batch_on()) st.push_back({[this, line, &batch] { run_batches(batch, line); }, 0, {}});
-      st.push_back({finish, 0, {1}});
-      return st;
+      return {{in_line, 0, {}},
+              {sums(0, qc_), 1, {0}},
+              {[this, line, &batch] { run_batches(batch, line); }, 0, {}},
+              {finish, 0, {1}}};
     }
     std::vector<Step> st{{load, 0, {}}, {decs, 2, {0}}, {zs(0, 1), 0, {}}, {sums(0, 1), 1, {2}}, {zs(1, 2), 0, {1}},
                          {sums(1, 2), 2, {4}}};
     int last = 5;  // the step that ends the second side stream
-    if (mid > 2) {
-      st.push_back({zs(2, mid), 0, {}});
-      st.push_back({sums(2, mid), 2, {6}});
+    if (qc_ > 2) {
+      st.push_back({zs(2, qc_), 0, {}});
+      st.push_back({sums(2, qc_), 2, {6}});
       last = 7;
     }
-    if (batch_on()) st.push_back({[this, &batch] { run_batches(batch, 1); }, 0, {}});
+    st.push_back({[this, &batch] { run_batches(batch, 1); }, 0, {}});
     st.push_back({finish, 0, {3, last}});
     return st;
   }
 
   // The reverse's steps.  Level n's gV and branch adjoint read only level-n
-  // fields and the prelude's operands, and write level-n buffers: they run on
-  // side streams (level 0's on one, the others', coarse to fine, on the other)
-  // beside the batched levels and the chains, which need the coarser chain
-  // and follow on the engine stream.
+  // fields and the prelude's operands, and write level-n buffers.  With
+  // batched levels they run on side streams (level 0's on one, the others',
+  // coarse to fine, on the other) beside the batched levels and the chains,
+  // which need the coarser chain and follow on the engine stream; without,
+  // levels 0 and 1's run on side streams beside the coarser levels' reverse.
   std::vector<Step> reverse_steps(double* grad_dev) {
     auto branches = [this](int from, int to) {  // coarse to fine
       return [this, from, to] {
@@ -1273,27 +1296,33 @@ class EngineT final : public Engine {
       };
     };
     if (levels_ == 1 || f_->recompute) return {{[this, grad_dev] { sweep_reverse(grad_dev); }, 0, {}}};
-    const int mid = batch_from();
-    if (few_steps()) {
-      std::vector<Step> st{{[this] { rev_prelude(); }, 0, {}}};
-      if (batch_on()) st.push_back({[this] { run_batches(qrev_); }, 0, {}});
-      st.push_back({branches(0, mid), 1, {0}});
-      st.push_back({[this, chains, mid, grad_dev] {
-                      chains(1, mid)();
-                      rev_chain(0, grad_dev);
-                    },
-                    0, {int(st.size()) - 1}});
-      return st;
+    auto prelude = [this] { rev_prelude(); };
+    auto last = [this, grad_dev] { rev_chain(0, grad_dev); };
+    if (!batch_on()) {
+      auto coarser = [this](int down_to) { return [this, down_to] { rev_levels(down_to); }; };
+      if (levels_ == 2) return {{prelude, 0, {}}, {branches(0, 1), 1, {0}}, {coarser(1), 0, {}}, {last, 0, {1}}};
+      return {{prelude, 0, {}},    {branches(0, 1), 1, {0}}, {branches(1, 2), 2, {0}},
+              {coarser(2), 0, {}}, {chains(1, 2), 0, {2}},   {last, 0, {1}}};
     }
-    std::vector<Step> st{{[this] { rev_prelude(); }, 0, {}}, {branches(0, 1), 1, {0}}};
-    if (mid > 2) st.push_back({branches(2, mid), 2, {0}});
+    auto batches = [this] { run_batches(qrev_); };
+    if (few_steps())
+      return {{prelude, 0, {}},
+              {batches, 0, {}},
+              {branches(0, qc_), 1, {0}},
+              {[this, chains, last] {
+                 chains(1, qc_)();
+                 last();
+               },
+               0, {2}}};
+    std::vector<Step> st{{prelude, 0, {}}, {branches(0, 1), 1, {0}}};
+    if (qc_ > 2) st.push_back({branches(2, qc_), 2, {0}});
     const int coarse = int(st.size()) - 1;
     st.push_back({branches(1, 2), 2, {0}});
     const int one = int(st.size()) - 1;
-    if (batch_on()) st.push_back({[this] { run_batches(qrev_); }, 0, {}});
-    if (mid > 2) st.push_back({chains(2, mid), 0, {coarse}});
+    st.push_back({batches, 0, {}});
+    if (qc_ > 2) st.push_back({chains(2, qc_), 0, {coarse}});
     st.push_back({chains(1, 2), 0, {one}});
-    st.push_back({[this, grad_dev] { rev_chain(0, grad_dev); }, 0, {1}});
+    st.push_back({last, 0, {1}});
     return st;
   }
 

@@ -389,6 +389,32 @@ def test_sweep_schedules_match_eager_launches(nside, J, batch, batch_nside):
             np.testing.assert_array_equal(g.vjp(cots, generation=it), e.vjp(cots, generation=it))
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["plain", "masks", "cross"])
+@pytest.mark.parametrize("nside,J,batch,batch_nside", [(32, 2, 1, 16), (32, 2, 40, 16), (16, 3, 2, 0), (64, 5, 1, 16),
+                                                       (64, 5, 6, 16), (128, 3, 2, 16)])
+def test_sweep_schedules_of_every_kind_match_eager_launches(nside, J, batch, batch_nside, kind, precision):
+    """The same for masked, cross and mixed engines: without batched levels two levels take four
+    steps and more take six, at any size; with them, few steps or all."""
+    from stl_port import NativeEngine
+    if kind == "cross":
+        batch = (batch + 1) // 2
+    print(f"[gpu] schedule {kind} nside={nside} J={J} batch={batch} {precision}", flush=True)
+    rng = np.random.default_rng(25)
+    npix = 12 * nside * nside
+    opts = dict(batch=batch, precision=precision, batch_nside=batch_nside, conv_variant=0, cross=kind == "cross")
+    if kind == "masks":
+        opts["masks"] = np.stack([np.arange(npix) % 3 > 0, np.arange(npix) < npix // 2]).astype(float)
+    with NativeEngine(nside, J, **opts) as g, NativeEngine(nside, J, timing=True, **opts) as e:
+        for it in range(3):
+            x = rng.standard_normal((batch, 2, npix) if kind == "cross" else (batch, npix))
+            vg, ve = (m.forward(x, generation=it, moments=it == 1) for m in (g, e))
+            for a, b in zip(vg, ve):
+                np.testing.assert_array_equal(a, b)
+            cot = rng.standard_normal(vg[0].shape) + 1j * rng.standard_normal(vg[0].shape)
+            np.testing.assert_array_equal(g.vjp(cot, generation=it), e.vjp(cot, generation=it))
+
+
 @pytest.mark.parametrize("cross", [False, True])
 @pytest.mark.parametrize("nside,J", [(2, 1), (16, 4), (32, 5)])
 def test_gram_reverse_lane_groups_match_per_pixel(nside, J, cross):
