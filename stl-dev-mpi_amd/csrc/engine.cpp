@@ -295,10 +295,12 @@ class EngineT final : public Engine {
     std::vector<DevArray<T>> maps, M;
     std::vector<DevArray<C2>> z, br;
     // Reverse buffers: gbr / gzp / acc[0] hold level 0, gbr1 / gzp1 / acc[1]
-    // level 1, lgbr / lgzp / lchain the levels n >= 2 (each its own), so that
-    // every level's gV and branch adjoint can run beside the coarser levels'
-    // reverse.
-    DevArray<C2> gbr, gzp, gz, gbr1, gzp1;
+    // level 1, lgzp / lchain the levels n >= 2 (each its own), so that every
+    // level's gV and branch adjoint can run beside the coarser levels'
+    // reverse.  A level's branch adjoint is the only reader of its gbr: the
+    // levels 2 .. qc - 1, which take turns on a stream, have gbr2 in common,
+    // the batched ones lgbr of their own.
+    DevArray<C2> gbr, gzp, gz, gbr1, gzp1, gbr2;
     std::vector<DevArray<C2>> lgbr, lgzp;
     DevArray<T> acc[2], mg[2];
     std::vector<DevArray<T>> lchain;
@@ -573,7 +575,8 @@ class EngineT final : public Engine {
   C2* br_of(int n) { return f_->br[f_->recompute ? 0 : n].data(); }
   bool batched(int n) const { return n >= qc_ && batch_on(); }
   C2* gbr_of(int n) {
-    return n == 0 || f_->recompute ? f_->gbr.data() : n == 1 ? f_->gbr1.data() : f_->lgbr[n].data();
+    if (n == 0 || f_->recompute) return f_->gbr.data();
+    return n == 1 ? f_->gbr1.data() : n < f_->qc ? f_->gbr2.data() : f_->lgbr[n].data();
   }
   C2* gzp_of(int n) {
     return n == 0 || f_->recompute ? f_->gzp.data() : n == 1 ? f_->gzp1.data() : f_->lgzp[n].data();
@@ -790,69 +793,84 @@ class EngineT final : public Engine {
     f_ = std::make_shared<FieldSet>();
     f_->rows = B_;
     f_->recompute = choose_recompute();
-    const size_t live0 = device_bytes_live();
-    f_->maps.resize(levels_);
-    f_->z.resize(levels_);
-    f_->M.resize(levels_);
-    f_->br.resize(levels_);
-    for (int n = 0; n < levels_; ++n) {
-      int64_t N = N_[n];
-      f_->maps[n].resize(size_t(B_) * N);
-      f_->M[n].resize(size_t(n + 1) * B_ * N * kL);
-      if (n == 0 || !f_->recompute) {
-        f_->z[n].resize(size_t(B_) * kL * N);
-        f_->br[n].resize(size_t(n + 1) * B_ * kL * N * kL);
-      }
-    }
-    // Level 0 has the largest branch, z and modulus fields: (n + 1) / 4^n <= 1.
-    f_->gbr.resize(f_->br[0].size());
-    f_->gzp.resize(f_->z[0].size());
-    f_->gz.resize(f_->z[0].size());
-    f_->acc[0].resize(f_->M[0].size());
-    f_->mg[0].resize(f_->maps[0].size());
-    f_->mg[1].resize(f_->maps[0].size());
-    if (f_->recompute) {
-      if (levels_ > 1) f_->acc[1].resize(f_->M[0].size());
-      f_->bytes = device_bytes_live() - live0;
-      alloc_sums();
-      return;
-    }
-    if (levels_ > 1) {
-      f_->gbr1.resize(f_->br[1].size());
-      f_->gzp1.resize(f_->z[1].size());
-      f_->acc[1].resize(f_->M[1].size());
-    }
-    f_->lgbr.resize(levels_);
-    f_->lgzp.resize(levels_);
-    f_->lchain.resize(levels_);
-    for (int n = 2; n < levels_; ++n) {
-      f_->lgbr[n].resize(f_->br[n].size());
-      f_->lgzp[n].resize(f_->z[n].size());
-      f_->lchain[n].resize(f_->M[n].size());
-    }
     f_->qc = qc_;
-    f_->qgz.resize(levels_);
-    f_->qmg.resize(levels_);
-    for (int n = qc_; n < levels_; ++n) {
-      f_->qgz[n].resize(f_->z[n].size());
-      f_->qmg[n].resize(f_->maps[n].size());
-    }
+    const size_t live0 = device_bytes_live();
+    auto resize = [](auto& buffer, size_t n) { buffer.resize(n); };
+    if (f_->recompute) recompute_buffers(*f_, resize);
+    else keep_buffers(*f_, resize);
     f_->bytes = device_bytes_live() - live0;
     alloc_sums();
   }
 
-  // Bytes of the keep store's fields and reverse buffers (what allocate() makes).
-  size_t keep_field_bytes() const {
-    auto len = [&](int n) { return n < levels_ ? size_t(N_[n]) : size_t(0); };
-    size_t e = 0, c = 0;  // real and complex elements
+  // Elements of level n's fields.
+  size_t map_len(int n) const { return size_t(B_) * N_[n]; }
+  size_t z_len(int n) const { return size_t(B_) * kL * N_[n]; }
+  size_t mod_len(int n) const { return size_t(n + 1) * B_ * N_[n] * kL; }
+  size_t branch_len(int n) const { return size_t(n + 1) * B_ * kL * N_[n] * kL; }
+
+  // The buffers of both stores: use(buffer, elements).  Level 0 has the
+  // largest branch, z and modulus fields: (n + 1) / 4^n <= 1.
+  template <typename F>
+  void common_buffers(FieldSet& f, F&& use) const {
+    f.maps.resize(levels_);
+    f.z.resize(levels_);
+    f.M.resize(levels_);
+    f.br.resize(levels_);
     for (int n = 0; n < levels_; ++n) {
-      // maps, moduli and the chain; z, branches and their cotangents
-      e += size_t(B_) * len(n) * (1 + 2 * (n + 1) * kL);
-      c += size_t(B_) * len(n) * 2 * kL * (1 + (n + 1) * kL);
+      use(f.maps[n], map_len(n));
+      use(f.M[n], mod_len(n));
     }
-    c += size_t(B_) * kL * len(0);  // gz
-    e += 2 * size_t(B_) * len(0);   // mg
-    return e * sizeof(T) + c * sizeof(C2);
+    use(f.z[0], z_len(0));
+    use(f.br[0], branch_len(0));
+    use(f.gbr, branch_len(0));
+    use(f.gzp, z_len(0));
+    use(f.gz, z_len(0));
+    use(f.acc[0], mod_len(0));
+    use(f.mg[0], map_len(0));
+    use(f.mg[1], map_len(0));
+  }
+
+  template <typename F>
+  void recompute_buffers(FieldSet& f, F&& use) const {
+    common_buffers(f, use);
+    if (levels_ > 1) use(f.acc[1], mod_len(0));
+  }
+
+  template <typename F>
+  void keep_buffers(FieldSet& f, F&& use) const {
+    common_buffers(f, use);
+    f.lgbr.resize(levels_);
+    f.lgzp.resize(levels_);
+    f.lchain.resize(levels_);
+    f.qgz.resize(levels_);
+    f.qmg.resize(levels_);
+    for (int n = 1; n < levels_; ++n) {
+      use(f.z[n], z_len(n));
+      use(f.br[n], branch_len(n));
+    }
+    if (levels_ > 1) {
+      use(f.gbr1, branch_len(1));
+      use(f.gzp1, z_len(1));
+      use(f.acc[1], mod_len(1));
+    }
+    if (qc_ > 2 && levels_ > 2) use(f.gbr2, branch_len(2));
+    for (int n = 2; n < levels_; ++n) {
+      use(f.lgzp[n], z_len(n));
+      use(f.lchain[n], mod_len(n));
+    }
+    for (int n = qc_; n < levels_; ++n) {
+      use(f.lgbr[n], branch_len(n));
+      use(f.qgz[n], z_len(n));
+      use(f.qmg[n], map_len(n));
+    }
+  }
+
+  // Bytes of the keep store's fields and reverse buffers.
+  size_t keep_field_bytes() const {
+    FieldSet none;
+    size_t bytes = 0;
+    keep_buffers(none, [&](const auto& buffer, size_t n) { bytes += n * sizeof(*buffer.data()); });
+    return bytes;
   }
 
   // The field store: forced, or (auto) keep when the kept fields take at most

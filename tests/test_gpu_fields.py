@@ -122,3 +122,22 @@ def test_fp64_pair_at_nside_2048_recompute_equals_keep():
         torch.cuda.empty_cache()
     np.testing.assert_array_equal(res["recompute"][0], res["keep"][0])
     np.testing.assert_array_equal(res["recompute"][1], res["keep"][1])
+
+
+@pytest.mark.parametrize("nside,J,batch,batch_nside,precision", [(16, 1, 2, 16, "fp64"), (32, 5, 3, 0, "mixed"),
+                                                                 (64, 6, 2, 16, "fp64"), (16, 4, 1, 16, "mixed")])
+def test_keep_store_memory(nside, J, batch, batch_nside, precision):
+    """The keep store holds the fields, levels 0 and 1's cotangents, one branch cotangent for the
+    coarser levels that are not batched, a z part and a chain for every level, and all cotangents of
+    the batched levels."""
+    from stl_port import NativeEngine
+    npix = [batch * 12 * (nside >> n) ** 2 for n in range(J)]
+    first = next((n for n in range(2, J) if npix[n] <= 12 * batch_nside ** 2), J)  # the first batched level
+    z, mod, br = ([a * p for a, p in zip(s, npix)] for s in ([4] * J, [4 * n + 4 for n in range(J)],
+                                                             [16 * n + 16 for n in range(J)]))
+    real = sum(npix) + 2 * sum(mod) + 2 * npix[0] + sum(npix[first:])
+    cplx = 2 * sum(z) + sum(br) + z[0] + sum(br[:2]) + sum(br[2:first][:1]) + sum(br[first:]) + sum(z[first:])
+    print(f"[gpu] keep store nside={nside} J={J} batch={batch} batch_nside={batch_nside} {precision}", flush=True)
+    with NativeEngine(nside, J, batch=batch, batch_nside=batch_nside, precision=precision, fields="keep") as e:
+        got = e.info()["device_memory"]["fields_bytes"]
+    assert got == (real + 2 * cplx) * (8 if precision == "fp64" else 4)
