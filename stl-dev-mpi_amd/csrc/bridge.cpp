@@ -269,6 +269,9 @@ StlHandle* stlp_new(const char* config) {
     opt.batch_nside = int(v.integer("batch_nside", 16));
     if (opt.batch_nside < 0) fail("batch_nside must be nonnegative");
     if (opt.conv_variant < -1 || opt.conv_variant > 5) fail("conv_variant must be -1 or 0 to 5");
+    opt.conv_forward = int(v.integer("conv_forward", -1));
+    if (opt.conv_forward != -1 && (opt.conv_forward < 6 || opt.conv_forward > 9))
+      fail("conv_forward must be -1 or 6 to 9");
     auto h = std::make_unique<StlHandle>();
     h->engine = stl::Engine::create(opt);
     (void)scratch_address(opt.device);

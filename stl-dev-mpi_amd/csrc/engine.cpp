@@ -1363,6 +1363,11 @@ class EngineT final : public Engine {
             (adj ? conv_adj_has_variant<T>(NI, kConvFaces32) : conv_fwd_has_variant<T>(NI, kConvFaces32)))
           cands.push_back(kConvFaces32);
         if (op.order <= 6) cands.push_back(kConvSplit);
+        if (opt_.conv_forward >= 0 && op.tiled && !adj &&
+            conv_fwd_mfma_fits(op.order, NI, rows, opt_.conv_forward)) {
+          conv_var_[n][kind] = opt_.conv_forward;
+          continue;
+        }
         if (opt_.conv_variant >= 0) {
           bool ok = std::find(cands.begin(), cands.end(), opt_.conv_variant) != cands.end();
           conv_var_[n][kind] = ok ? opt_.conv_variant : kConvTiled;

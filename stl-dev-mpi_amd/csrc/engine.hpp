@@ -45,6 +45,10 @@ struct EngineOptions {
   // and kernel by timing at creation (cached per device, precision, level and
   // shape); 0, 1, 2 force one where the kernel has it (see sweeps.hpp).
   int conv_variant = -1;
+  // Matrix-core form of the forward convolutions (6 to 9, see sweeps.hpp)
+  // wherever it fits the level and its rows, before any other choice; -1: by
+  // timing as the others.
+  int conv_forward = -1;
   // What the forward keeps for the reverse (the reference's FieldStore,
   // crates/stl-gpu/src/engine.rs:172-186): keep stores every level's z and
   // branches; recompute stores the maps and moduli only and recomputes each

@@ -15,7 +15,7 @@ Maps and gradients on the device (torch tensors or raw addresses) go through the
 methods without host copies.  The library has no CPU path and this module has no fallback: a
 missing library raises at construction.  Keywords of this library beyond the reference's:
 `precision` ("fp64" | "mixed"), `fields` ("keep" | "recompute" | "auto"), `timing`,
-`conv_variant`, `families`, `batch_nside` (levels of at most this nside run batched, each step
+`conv_variant`, `conv_forward`, `families`, `batch_nside` (levels of at most this nside run batched, each step
 of a sweep one launch for all of them; 0: none).
 """
 from __future__ import annotations
@@ -277,7 +277,8 @@ class NativeEngine:
     def __init__(self, nside, j, batch=1, backend="gpu", kernel=5, orientations=4, block_pixels=4096,
                  cache_bytes=1 << 30, threads=1, cache="transposition", device=0, library=None, cross=False,
                  masks=None, spin=0, spin_kernel=5, spin_pyramid="scalar", spin_a=2, precision="fp64",
-                 fields="auto", timing=False, conv_variant=None, families=None, batch_nside=None):
+                 fields="auto", timing=False, conv_variant=None, families=None, batch_nside=None,
+                 conv_forward=None):
         self._lock = threading.RLock()
         self._h = None
         self._lib = bridge(library)
@@ -298,6 +299,8 @@ class NativeEngine:
                       cross=bool(cross), spin=int(spin), precision=precision, fields=fields, timing=bool(timing))
         if conv_variant is not None:
             config["conv_variant"] = int(conv_variant)
+        if conv_forward is not None:
+            config["conv_forward"] = int(conv_forward)
         if families is not None:
             config["families"] = ",".join(families)
         if batch_nside is not None:

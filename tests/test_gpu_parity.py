@@ -618,3 +618,36 @@ def test_matrix_core_forward_agrees_with_the_tiled_one(nside, J, batch, precisio
     # Rounding of 50 slots' sums, twice (z and its modulus' wavelets), a product and J levels.
     eps = (2.0 ** -24 if precision == "mixed" else 2.0 ** -53) * 50 * 4 * (J + 1)
     assert np.abs(v1 - v0).max() <= eps * np.abs(v0).max()
+
+
+@pytest.mark.parametrize("form", [6, 7, 8, 9])
+@pytest.mark.parametrize("nside,J,batch,precision", [(8, 1, 3, "fp64"), (8, 1, 3, "mixed"), (16, 2, 1, "fp64"), (16, 2, 1, "mixed"),
+                                                     (32, 3, 3, "fp64"), (32, 3, 3, "mixed"), (64, 3, 2, "mixed")])
+def test_every_matrix_core_form_agrees_with_the_tiled_one(nside, J, batch, precision, form):
+    """Each form of the matrix-core forward (8 x 8 tiles with 1 or 2 rows per workgroup, 16 x 16 with 1
+    or 2), forced on every level that it fits, against the 16 x 16 thread-per-pixel form: one row, odd
+    rows (a last group of one), faces of one tile.  FP32: the same bits of statistics and gradients, also
+    of maps of denormal numbers.  FP64: a z or branch value sums 44 products in another order, each within
+    2^-53 of the terms' sum, and a coefficient holds a product of two of them averaged over pixels, one
+    decimation (32 products) per level above it."""
+    from stl_port import NativeEngine
+    rng = np.random.default_rng(nside + batch)
+    opts = dict(batch=batch, precision=precision, conv_variant=0, batch_nside=0)
+    with NativeEngine(nside, J, conv_forward=form, **opts) as m, NativeEngine(nside, J, **opts) as t:
+        for n, (z, branch, *adjoints) in enumerate(m.info()["conv_variants"]):
+            fits = lambda wide, rows: ((nside >> n) >= (8 if form < 8 else 16) and (form % 2 == 0 or rows >= 2)
+                                       and not (wide and form == 7))
+            assert z == (form if fits(False, batch) else 0) and branch == (form if fits(True, (n + 1) * batch) else 0)
+            assert adjoints == [0, 0]
+        for scale in (1.0, 2.0 ** -132) if precision == "mixed" else (1.0,):
+            print(f"[gpu] matrix-core form {form} nside={nside} J={J} B={batch} {precision} {scale}", flush=True)
+            x = scale * rng.standard_normal((batch, 12 * nside * nside))
+            (vm, sm), (vt, st) = (e.forward(x, moments=True) for e in (m, t))
+            cot = rng.standard_normal(vt.shape) + 1j * rng.standard_normal(vt.shape)
+            gm, gt = (e.vjp(cot) for e in (m, t))
+            if precision == "mixed":
+                for a, b in ((vm, vt), (sm, st), (gm, gt)):
+                    np.testing.assert_array_equal(a, b)
+            else:
+                eps = 2.0 ** -53 * (2 * 2 * 44 + 32 * (J - 1))
+                assert np.abs(vm - vt).max() <= eps * np.abs(vt).max()

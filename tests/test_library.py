@@ -74,6 +74,13 @@ def test_bad_configuration_is_an_error(config, message):
         lib.call("stlp_new", config.encode())
 
 
+@pytest.mark.parametrize("form", [-2, 0, 5, 10])
+def test_matrix_core_form_outside_its_table_is_an_error(form):
+    lib = native.bridge()
+    with pytest.raises(native.BridgeError, match="conv_forward"):
+        lib.call("stlp_new", json.dumps({"nside": 16, "j": 3, "conv_forward": form}).encode())
+
+
 def test_other_products_are_not_implemented():
     lib = native.bridge().cdll
     assert not lib.stlp_patch_new(b"{}")
