@@ -1346,8 +1346,9 @@ class EngineT final : public Engine {
 
   // Convolution kernel variant per level and kernel (forward z, forward
   // branch, adjoint z, adjoint branch): forced, or the fastest of the
-  // candidates timed on this level's operator and buffers (a candidate must
-  // beat the default by 3%), remembered for the process.
+  // candidates timed on this level's operator and buffers (among the forms
+  // without matrix cores one must beat the first by 3%; a matrix-core form
+  // only has to be faster), remembered for the process.
   void tune() {
     conv_var_.assign(levels_, {kConvTiled, kConvTiled, kConvTiled, kConvTiled});
     for (int n = 0; n < levels_; ++n) {
@@ -1394,7 +1395,11 @@ class EngineT final : public Engine {
           return time_launch([&] { launch_conv_adj<T>(op, NI, gy, rows, gx, s_, v); });
         };
         // The forward's matrix-core variants replace the others on tiled
-        // levels (FP64: 1.5 to 2 times faster at every size).  In FP32 they
+        // levels.  FP64: branches are 1.1 to 2.1 times as fast, maps 1.2 to
+        // 2.9 times (several rows, or up to nside 128), but one row of maps is
+        // bound by its coefficients in both forms (us, several faces /
+        // matrix-core, nside 256 107 / 108, 512 391 / 377, 1024 1484 / 1434,
+        // 2048 5584 / 5727): from nside 2048 on both are timed.  In FP32 they
         // add a row's slots in the same order as the tiled ones but not as
         // the split one, whose choice is made among the older variants; from
         // nside 128 on, where it is no candidate, only the older ones that
@@ -1404,7 +1409,8 @@ class EngineT final : public Engine {
           for (int v = kConvMfma; v < kConvMfma + kFwdMfmas; ++v)
             if (conv_fwd_mfma_fits(op.order, NI, rows, v)) more.push_back(v);
         if (!more.empty()) {
-          if (sizeof(T) == 8) cands.clear();
+          if (sizeof(T) == 8)
+            cands = NI == 1 && rows == 1 && op.order >= 11 ? std::vector<int>{kConvFaces} : std::vector<int>{};
           else if (op.order > 6) cands = NI == 1 ? std::vector<int>{kConvFaces, kConvFaces32} : std::vector<int>{kConvFaces32};
         }
         // Two interleaved rounds, each candidate's best: no bias from the

@@ -9,6 +9,11 @@ statistics 1e-13 per family (max |dS| / max |S|), variances 1e-12, gradient
 held to 1e-5 per family and 1e-4 on the gradient at these small sizes; its
 error at the benchmark's size is checked against oracle vectors elsewhere.
 """
+import json
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -17,6 +22,8 @@ import oracle as O
 from fixtures import cases
 
 pytestmark = pytest.mark.gpu
+
+ROOT = Path(__file__).resolve().parents[1]
 
 torch = pytest.importorskip("torch")
 
@@ -651,3 +658,19 @@ def test_every_matrix_core_form_agrees_with_the_tiled_one(nside, J, batch, preci
             else:
                 eps = 2.0 ** -53 * (2 * 2 * 44 + 32 * (J - 1))
                 assert np.abs(vm - vt).max() <= eps * np.abs(vt).max()
+
+
+def test_one_row_of_large_maps_is_timed_with_and_without_matrix_cores():
+    """One FP64 map at nside 2048: the several-face form (variant 1) is a little faster than the
+    matrix-core ones, so the choice times both.  In a process of its own: a choice is made once per process."""
+    code = ("import json, sys; sys.path.insert(0, sys.argv[1]); from stl_port import NativeEngine\n"
+            "with NativeEngine(2048, 2, precision='fp64') as e: print(json.dumps(e.info()['conv_tuning']))")
+    print("[gpu] tuning candidates nside=2048 fp64", flush=True)
+    out = subprocess.run([sys.executable, "-c", code, str(ROOT / "stl-dev-mpi_amd")], capture_output=True, text=True,
+                         timeout=100, check=True)
+    timed = {(level, kind): set() for level in range(2) for kind in range(4)}
+    for level, kind, variant, _ in json.loads(out.stdout.splitlines()[-1]):
+        timed[level, kind].add(variant)
+    assert timed[0, 0] == {1, 6, 8}
+    assert timed[0, 1] == {6, 8}  # branches: the matrix-core forms alone
+    assert timed[1, 0] == {6, 8}  # nside 1024
